@@ -10,7 +10,9 @@ namespace compas {
 
 namespace kernels {
 struct FispArgs;
+struct PssfpArgs;
 struct PssfpTableJob;
+struct PssfpMapArgs;
 }  // namespace kernels
 
 // dst[i] += src[i] for i < n (complex)
@@ -151,6 +153,25 @@ void launch_fisp_table(const CompasContext& ctx, int spl, const kernels::FispArg
 int pssfp_table_zpl(int nz);
 void launch_pssfp_table(
     const CompasContext& ctx, int zpl, const kernels::PssfpTableJob* jobs, const int4* items, int n);
+
+// The simulation by one affine map per isochromat and TR (pssfp_map.hip):
+// whether it pays for a train; the doubles of the train's table; the launch
+// arguments, with the table's kernel enqueued (`zpl`: slice positions per lane
+// of the sub-step form, should the train be beyond the maps); the partial
+// planes that either form needs; the workgroups of the maps, launched for one
+// simulation (jobs == nullptr) or as items (job, unit) of a work table; the
+// sub-step form, which does nothing where the maps served; and what follows
+// the maps: that form and the sum of the partial planes.
+bool pssfp_map_pays(int nTR, int nRF);
+int64_t pssfp_map_train_size(int nTR);
+void pssfp_map_setup(const CompasContext& ctx, kernels::PssfpMapArgs& p, const kernels::PssfpArgs& a, double* train, int zpl);
+int pssfp_map_partial_planes(const kernels::PssfpMapArgs& p);
+int64_t pssfp_map_units(const kernels::PssfpMapArgs& p);
+void launch_pssfp_map(
+    const CompasContext& ctx, const kernels::PssfpMapArgs& single, const kernels::PssfpMapArgs* jobs,
+    const int2* items, int64_t n);
+void launch_pssfp_unmapped(const CompasContext& ctx, const kernels::PssfpMapArgs& p);
+void pssfp_map_finish(const CompasContext& ctx, const kernels::PssfpMapArgs& p);
 
 // Finite-difference pieces of simulate_magnetization_derivative
 // (derivative.cu:11-94): the parameters with `field` moved by `delta` (the

@@ -1,4 +1,6 @@
-// pSSFP isochromat (Bloch) simulation on gfx950.
+// pSSFP isochromat (Bloch) simulation on gfx950, RF sub-step by RF sub-step:
+// the form for short trains and waveforms and for flip angles beyond the per-TR
+// maps (pssfp_map.hip), which carry the others.
 //
 // Semantics: reference src/simulate/pssfp_kernels.cuh:14-129, pssfp.cu:7-91
 // and src/operators/isochromat.cuh:9-128.
@@ -37,6 +39,7 @@
 
 #include "compas/device/common.h"
 #include "compas/device/pssfp_common.h"
+#include "compas/device/pssfp_map.h"
 #include "compas/internal.h"
 
 namespace compas {
@@ -197,9 +200,11 @@ __device__ __forceinline__ void pssfp_iso_block(const PssfpArgs& a, int group, i
 
 // grid (ceil(nv / 64), groups in this launch), block 64.  Group g of the
 // launch is group0 + blockIdx.y; blockIdx.y == 0 writes out0, blockIdx.y = j
-// > 0 writes rest + (j - 1) * nTR * nv.
+// > 0 writes rest + (j - 1) * nTR * nv.  train: nullptr, or the table of a
+// train (pssfp_map.h); the launch does nothing where the maps served it.
 template<int ZPL>
-__global__ void __launch_bounds__(64) pssfp_iso(PssfpArgs a, int group0, cfloat* out0, cfloat* rest) {
+__global__ void __launch_bounds__(64) pssfp_iso(PssfpArgs a, int group0, cfloat* out0, cfloat* rest, const double* train) {
+    if (train != nullptr && train[1] != 0.0) return;
     __shared__ double2 grf[RF_CHUNK];  // gamma_dt_RF as doubles (LDS broadcast reads)
     const size_t plane = size_t(a.nTR) * size_t(a.tissue.nvoxels);
     cfloat* out = (blockIdx.y == 0) ? out0 : rest + size_t(blockIdx.y - 1) * plane;
@@ -283,11 +288,12 @@ PssfpLayout pssfp_layout(const CompasContext& ctx, int nz, int nv, int nTR, cons
 
 namespace {
 
-using PssfpLauncher = void (*)(kernels::PssfpArgs, int, cfloat*, cfloat*, dim3, hipStream_t);
+using PssfpLauncher = void (*)(kernels::PssfpArgs, int, cfloat*, cfloat*, const double*, dim3, hipStream_t);
 
 template<int ZPL>
-void launch_pssfp(kernels::PssfpArgs a, int group0, cfloat* out0, cfloat* rest, dim3 grid, hipStream_t s) {
-    kernels::pssfp_iso<ZPL><<<grid, 64, 0, s>>>(a, group0, out0, rest);
+void launch_pssfp(
+    kernels::PssfpArgs a, int group0, cfloat* out0, cfloat* rest, const double* train, dim3 grid, hipStream_t s) {
+    kernels::pssfp_iso<ZPL><<<grid, 64, 0, s>>>(a, group0, out0, rest, train);
 }
 
 PssfpLauncher pssfp_launcher(int zpl) {
@@ -313,6 +319,13 @@ int resident_waves() {
 }
 
 }  // namespace
+
+void launch_pssfp_unmapped(const CompasContext& ctx, const kernels::PssfpMapArgs& p) {
+    KernelScope ks(ctx, "pssfp_iso");
+    const dim3 grid(dev::div_ceil(p.a.tissue.nvoxels, 64), unsigned(p.direct_groups));
+    pssfp_launcher(p.direct_zpl)(p.a, 0, p.a.echos, p.partial, p.train, grid, ctx.stream());
+    check_launch("pssfp_iso");
+}
 
 int pssfp_table_zpl(int nz) {
     // the fewest groups of at most 7 positions, balanced: 35 -> 7 x 5, 10 -> 5 x 2
@@ -396,6 +409,19 @@ Array<cfloat, 2> simulate_magnetization(
 
     const PssfpLayout L = primal_layout(ctx, nz, nv, nTR);
     const int64_t plane = int64_t(nTR) * nv;
+    // by maps where they pay and the sub-step form they fall back to would run
+    // as one launch
+    if (pssfp_map_pays(nTR, a.nRF) && L.groups <= L.per_launch) {
+        auto train = ctx.empty<double, 1>({pssfp_map_train_size(nTR)});
+        kernels::PssfpMapArgs p;
+        pssfp_map_setup(ctx, p, a, train.data(), L.zpl);
+        Array<cfloat, 2> part;
+        if (const int planes = pssfp_map_partial_planes(p)) part = ctx.empty<cfloat, 2>({planes, plane});
+        p.partial = part.data();
+        launch_pssfp_map(ctx, p, nullptr, nullptr, pssfp_map_units(p));
+        pssfp_map_finish(ctx, p);
+        return echos;
+    }
     const int slots = partial_slots(L);
     Array<cfloat, 2> part;
     if (slots > 0) part = ctx.empty<cfloat, 2>({slots, plane});
@@ -407,7 +433,7 @@ Array<cfloat, 2> simulate_magnetization(
         cfloat* rest = g0 == 0 ? part.data() : part.data() + plane;
         {
             KernelScope ks(ctx, "pssfp_iso");
-            fn(a, g0, out0, rest, dim3(vblocks, unsigned(count)), ctx.stream());
+            fn(a, g0, out0, rest, nullptr, dim3(vblocks, unsigned(count)), ctx.stream());
             check_launch("pssfp_iso");
         }
         pssfp_sum_groups(ctx, echos.data(), part.data(), g0 == 0 ? count - 1 : count, plane, plane);

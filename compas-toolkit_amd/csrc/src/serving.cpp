@@ -8,8 +8,8 @@
 //      FISP RF tables, pSSFP partial planes, perturbed tissue copies) comes
 //      from the pool of sim_[0], set up on its stream after the request's
 //      inputs are ready.
-//   2. Work-table launches.  Each launch takes up to batch_waves() work items
-//      (one wave each) from the active jobs, least GPU time used first (each
+//   2. Work-table launches.  Each launch takes up to batch_items() work items
+//      (a wave, or a workgroup of the pSSFP maps) from the active jobs, least GPU time used first (each
 //      job's virtual time grows by its item cost), groups them by kernel
 //      instance and launches fisp_epg_table / pssfp_iso_table over a table
 //      uploaded from pinned memory.  Launches alternate over two streams with
@@ -34,6 +34,7 @@
 
 #include "compas/device/fisp_common.h"
 #include "compas/device/pssfp_common.h"
+#include "compas/device/pssfp_map.h"
 #include "compas/internal.h"
 
 namespace compas {
@@ -48,14 +49,16 @@ constexpr float kDelta = 1e-4f;  // finite-difference step (derivative.h:21-47 d
 // (measured on the simulate + signal steps of 50176 voxels x 1120 TRs: 2.26
 // ms per step with 1024, 2.38 with 2048).  COMPAS_SERVER_BATCH_WAVES sets
 // both (measurement).
-int batch_waves(bool pssfp) {
+// pSSFP by maps: 1024 workgroups, two rounds of the two that a CU holds, each
+// round 0.4 ms for a train of 1000 TRs.
+int batch_items(bool pssfp, bool maps) {
     static const int forced = [] {
         const char* e = std::getenv("COMPAS_SERVER_BATCH_WAVES");
         const int v = e ? std::atoi(e) : 0;
         return v >= 64 && v <= 65536 ? v : 0;
     }();
     if (forced) return forced;
-    return pssfp ? 2048 : 1024;
+    return pssfp && !maps ? 2048 : 1024;
 }
 
 constexpr int kMaxBatchJobs = 256;  // simulations per launch
@@ -137,6 +140,7 @@ struct Server::SimJob {
     size_t index = 0;  // position in the request's jobs (0: the echoes)
     int field = -1;  // finite-difference field of this job, -1 for the echoes
     bool pssfp = false;
+    bool maps = false;  // pSSFP by per-TR maps (pssfp_map.hip); an item is one of its units
     int bucket = 0;  // kernel instance: FISP states per lane, pSSFP slice positions per lane
     int vblocks = 0, groups = 1;
     int64_t items = 0, next = 0;  // work items, and the first not yet launched
@@ -145,8 +149,10 @@ struct Server::SimJob {
     TissueParameters params;  // the request's, or the perturbed copy
     kernels::FispArgs fisp {};
     kernels::PssfpTableJob pss {};
+    kernels::PssfpMapArgs map {};
     Array<cfloat, 2> echos, partial;
     Array<float4, 1> table;
+    Array<double, 1> train;
     std::shared_ptr<Event> last[Server::kSimStreams];  // last launch holding items of this job, per stream
 };
 
@@ -207,7 +213,7 @@ std::shared_ptr<Server::SimJob> make_job(const CompasContext& sim, const ServeRe
             j->bucket = zpl;
             j->groups = (nz + zpl - 1) / zpl;
             const int64_t plane = int64_t(nTR) * nv;
-            if (j->groups > 1) j->partial = sim.empty<cfloat, 2>({j->groups - 1, plane});
+            j->maps = pssfp_map_pays(nTR, nRF);
             kernels::PssfpArgs& a = j->pss.a;
             a.tissue = dev::tissue_view(j->params);
             a.RF = seq.RF_train.data();
@@ -222,6 +228,17 @@ std::shared_ptr<Server::SimJob> make_job(const CompasContext& sim, const ServeRe
             a.g_ex = seq.gamma_dt_GRz.ex;
             a.g_pr = seq.gamma_dt_GRz.pr;
             a.echos = j->echos.data();
+            if (j->maps) {
+                j->train = sim.empty<double, 1>({pssfp_map_train_size(nTR)});
+                pssfp_map_setup(sim, j->map, a, j->train.data(), zpl);
+                if (const int planes = pssfp_map_partial_planes(j->map)) j->partial = sim.empty<cfloat, 2>({planes, plane});
+                j->map.partial = j->partial.data();
+                j->items = pssfp_map_units(j->map);
+                j->bucket = 0;  // one kernel instance for all
+                j->item_cost = 4.0 * (100.0 * nTR + 700.0 * nRF);
+                return j;
+            }
+            if (j->groups > 1) j->partial = sim.empty<cfloat, 2>({j->groups - 1, plane});
             j->pss.partial = j->partial.data();
             j->items = int64_t(j->vblocks) * j->groups;
             j->item_cost = double(nTR + 1) * std::max(nRF, 1) * (zpl * 50.0 + 12.0) + double(nTR) * zpl * 40.0;
@@ -288,7 +305,7 @@ size_t Server::estimate_bytes(const ServeRequest& r) const {
         const int nz = int(r.pssfp->z.size(0));
         if (nz > 0) {
             const int zpl = pssfp_table_zpl(nz);
-            bytes += size_t((nz + zpl - 1) / zpl - 1) * echo;
+            bytes += size_t((nz + zpl - 1) / zpl - 1) * echo;  // (the maps need no more planes)
         }
     }
     if (r.kind == RequestKind::SimulateSignal) {
@@ -439,7 +456,9 @@ void Server::complete_jobs() {
             for (int st = 1; st < kSimStreams; st++) {
                 if (j.last[st]) COMPAS_HIP_CHECK(hipStreamWaitEvent(sim.stream(), j.last[st]->ev, 0));
             }
-            if (j.pssfp && j.groups > 1) {
+            if (j.maps) {
+                pssfp_map_finish(sim, j.map);
+            } else if (j.pssfp && j.groups > 1) {
                 const int64_t plane = j.echos.numel();
                 pssfp_sum_groups(sim, j.echos.data(), j.partial.data(), j.groups - 1, plane, plane);
             }
@@ -494,17 +513,18 @@ void Server::build_and_launch_batch() {
     }
     if (best < 0) return;
     const bool want_pssfp = active_jobs_[size_t(best)]->pssfp;
+    const bool want_maps = active_jobs_[size_t(best)]->maps;
     const int want_bucket = active_jobs_[size_t(best)]->bucket;
     using Key = std::pair<double, size_t>;
     std::priority_queue<Key, std::vector<Key>, std::greater<Key>> heap;
     for (size_t i = 0; i < active_jobs_.size(); i++) {
         const SimJob& j = *active_jobs_[i];
-        if (j.next < j.items && j.pssfp == want_pssfp && j.bucket == want_bucket) heap.push({j.vtime, i});
+        if (j.next < j.items && j.pssfp == want_pssfp && j.maps == want_maps && j.bucket == want_bucket) heap.push({j.vtime, i});
     }
     std::vector<int> local(active_jobs_.size(), -1);  // job -> index among this launch's jobs
     std::vector<size_t> jobs;  // active_jobs_ indices in the launch
     std::vector<std::pair<size_t, int64_t>> picks;  // (launch job, item)
-    const int max_items = batch_waves(want_pssfp);
+    const int max_items = batch_items(want_pssfp, want_maps);
     while (!heap.empty() && int(picks.size()) < max_items) {
         const size_t i = heap.top().second;
         heap.pop();
@@ -528,7 +548,7 @@ void Server::build_and_launch_batch() {
     // table layout: per kernel instance (FISP states / pSSFP positions per
     // lane) its job descriptors, then its items
     struct Instance {
-        bool pssfp;
+        bool pssfp, maps;
         int bucket;
         std::vector<int> job_ids;  // launch jobs of this instance
         std::vector<int> slot_of;  // launch job -> descriptor index in this instance
@@ -541,10 +561,10 @@ void Server::build_and_launch_batch() {
         const SimJob& j = *active_jobs_[jobs[lj]];
         int found = -1;
         for (size_t q = 0; q < inst.size(); q++) {
-            if (inst[q].pssfp == j.pssfp && inst[q].bucket == j.bucket) found = int(q);
+            if (inst[q].pssfp == j.pssfp && inst[q].maps == j.maps && inst[q].bucket == j.bucket) found = int(q);
         }
         if (found < 0) {
-            inst.push_back({j.pssfp, j.bucket, {}, std::vector<int>(jobs.size(), -1), 0, 0, 0});
+            inst.push_back({j.pssfp, j.maps, j.bucket, {}, std::vector<int>(jobs.size(), -1), 0, 0, 0});
             found = int(inst.size()) - 1;
         }
         inst_of[lj] = found;
@@ -555,16 +575,20 @@ void Server::build_and_launch_batch() {
     size_t off = 0;
     for (auto& q : inst) {
         q.jobs_off = off;
-        off = align16(off + q.job_ids.size() * (q.pssfp ? sizeof(kernels::PssfpTableJob) : sizeof(kernels::FispArgs)));
+        off = align16(off + q.job_ids.size() * (q.maps ? sizeof(kernels::PssfpMapArgs)
+                                                   : q.pssfp ? sizeof(kernels::PssfpTableJob)
+                                                             : sizeof(kernels::FispArgs)));
         q.items_off = off;
-        off = align16(off + size_t(q.nitems) * (q.pssfp ? sizeof(int4) : sizeof(int2)));
+        off = align16(off + size_t(q.nitems) * (q.pssfp && !q.maps ? sizeof(int4) : sizeof(int2)));
     }
     COMPAS_CHECK(off <= kRingBytes);
     char* host = static_cast<char*>(host_ring_[ring]);
     for (auto& q : inst) {
         for (size_t d = 0; d < q.job_ids.size(); d++) {
             const SimJob& j = *active_jobs_[jobs[size_t(q.job_ids[d])]];
-            if (q.pssfp) {
+            if (q.maps) {
+                std::memcpy(host + q.jobs_off + d * sizeof(kernels::PssfpMapArgs), &j.map, sizeof(j.map));
+            } else if (q.pssfp) {
                 std::memcpy(host + q.jobs_off + d * sizeof(kernels::PssfpTableJob), &j.pss, sizeof(j.pss));
             } else {
                 std::memcpy(host + q.jobs_off + d * sizeof(kernels::FispArgs), &j.fisp, sizeof(j.fisp));
@@ -580,7 +604,7 @@ void Server::build_and_launch_batch() {
         tickets.insert(j.ticket);
         const int d = q.slot_of[p.first];
         const int n = fill[qi]++;
-        if (q.pssfp) {
+        if (q.pssfp && !q.maps) {
             const int vb = int(p.second % j.vblocks), g = int(p.second / j.vblocks);
             reinterpret_cast<int4*>(host + q.items_off)[n] = make_int4(d, vb, g, 0);
         } else {
@@ -594,7 +618,10 @@ void Server::build_and_launch_batch() {
     uint8_t* dev = dev_ring_[ring].data();
     COMPAS_HIP_CHECK(hipMemcpyAsync(dev, host, off, hipMemcpyHostToDevice, ctx.stream()));
     for (auto& q : inst) {
-        if (q.pssfp) {
+        if (q.maps) {
+            launch_pssfp_map(ctx, {}, reinterpret_cast<const kernels::PssfpMapArgs*>(dev + q.jobs_off),
+                             reinterpret_cast<const int2*>(dev + q.items_off), q.nitems);
+        } else if (q.pssfp) {
             launch_pssfp_table(ctx, q.bucket, reinterpret_cast<const kernels::PssfpTableJob*>(dev + q.jobs_off),
                                reinterpret_cast<const int4*>(dev + q.items_off), q.nitems);
         } else {

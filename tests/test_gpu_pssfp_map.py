@@ -1,0 +1,58 @@
+"""pSSFP by one affine map per isochromat and TR (pssfp_map.hip) against the
+FP64 oracle, where its layout or its choice of form changes: workgroups of one
+and of many voxels, a last voxel block and a last TR chunk that are not full,
+several slice-position groups, trains with RF phases, trains too strong for the
+maps, and trains too short for them.
+
+Tolerance: the state is FP64 throughout and the maps leave at most 2e-12 per
+TR, so what remains is one FP32 rounding of each echo and one of each partial
+plane (at most 4 here): 5 x 6e-8 = 3e-7.
+"""
+
+import numpy as np
+import pytest
+
+import compas_amd as ca
+from compas_amd import workloads as W
+from gpu_helpers import banner, context, rel
+
+pytestmark = pytest.mark.gpu
+
+TOL = 3e-7
+
+
+def train(nTR, deg, nz, nRF, phase):
+    seq = W.make_pssfp(nTR, deg, nz=nz, nRF=nRF)
+    if phase:
+        seq.RF = (seq.RF * np.exp(1j * phase * np.sin(np.arange(nTR)))).astype(np.complex64)
+    if nz > 1:
+        # a gradient that dephases the slice during the pulse as well
+        seq.gamma_dt_GRz = (1.5 / nRF, 0.0, -0.75)
+    return seq
+
+
+@pytest.mark.parametrize("nv,nTR,nz,nRF,deg,phase", [
+    (1, 65, 1, 12, 60.0, 0.0),       # one isochromat
+    (257, 64, 1, 25, 70.0, 0.0),     # 256 voxels to a workgroup, then one
+    (15, 71, 35, 25, 70.0, 0.0),     # 7 voxels to a workgroup; 71 = 8 x 8 + 7 TRs
+    (15, 71, 35, 25, 70.0, 1.1),     # the same with RF phases
+    (6, 72, 128, 9, 45.0, 0.7),      # the most slice positions of one group
+    (5, 66, 131, 8, 45.0, 0.0),      # two groups
+    (70, 64, 35, 25, 170.0, 0.4),    # too strong for the maps: sub-steps, by waves
+    (3, 80, 10, 256, 60.0, 0.0),     # the longest waveform that is staged whole
+    (3, 80, 10, 257, 60.0, 0.0),     # one more: sub-steps
+    (40, 30, 35, 25, 70.0, 0.0),     # too few TRs: sub-steps
+    (9, 100, 11, 25, 0.0, 0.0),      # no flip at all
+])
+def test_pssfp_map(oracle, nv, nTR, nz, nRF, deg, phase):
+    banner(f"pssfp map {nv} voxels {nTR} TRs {nz} positions {nRF} sub-steps {deg} deg phase {phase}")
+    context()
+    n = int(np.ceil(np.sqrt(nv)))
+    t = W.make_tissue(W.SplitMix64(77), n, 20.0, 40.0).slice(0, nv)
+    seq = train(nTR, deg, nz, nRF, phase)
+    got = ca.simulate_magnetization(ca.TissueParameters.from_tissue(t), ca.pSSFPSequence.from_sequence(seq)).collect()
+    want = oracle.pssfp(t, seq, "f64")
+    if deg == 0.0:
+        assert np.array_equal(got, np.zeros_like(got))
+    else:
+        assert rel(got, want) < TOL
