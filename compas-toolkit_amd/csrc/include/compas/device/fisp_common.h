@@ -10,7 +10,10 @@ namespace kernels {
 
 struct FispArgs {
     dev::TissueView tissue;
-    const float4* table;  // [nslices][nTR]: (deg2rad*|RF|, cos phi, sin phi, 0), then one zero entry
+    // [nslices][nTR]: (deg2rad*|RF|, cos phi, sin phi, 0); then (the largest
+    // deg2rad*|RF|, 0, 0, 1 if every sin phi is 0 and else 0), then one more
+    // entry, so that a recursion may load two entries ahead
+    const float4* table;
     int nTR;
     int nslices;
     float TR, TE, TW, TI;
@@ -34,16 +37,10 @@ __device__ inline cfloat off_resonance(float dt, float B0) {
     return {c, s};
 }
 
-// Largest flip angle (deg2rad |RF|) of the launch's RF table, the same in
-// every lane of the wave.  Every lane of the wave must be active.
-__device__ inline float fisp_table_max_angle(const FispArgs& a) {
-    const int total = a.nslices * a.nTR;
-    float m = 0.0f;
-    for (int i = int(__lane_id()); i < total; i += 64) m = fmaxf(m, fabsf(a.table[i].x));
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-    return m;
-}
+// Planes that a tangent pass writes, in the order of TangentSet
+struct FispPlanes {
+    cfloat* p[5];  // [nTR * usf][nvoxels] each
+};
 
 // Forms of the half flip angle's sincos in the TR loop
 enum FispHalfAngle : int {
@@ -79,21 +76,24 @@ __device__ inline bool fisp_direct_echo(const FispArgs& a, float T2, float B0) {
 // half flip angles alpha/2 = t.x B1 / 2 of the wave are bounded by h = 0.5
 // fl(max_angle |B1|), since rounding is monotone (|fl(t.x B1)| <=
 // fl(max_angle |B1|)).  wide: h may exceed 64, where sincos_fast leaves its
-// polynomial; q0: fl(h 2/pi) <= 1/2, every reduction index is 0; simple: one
-// slice profile, one repetition, no undersampling, no direct echo and at
-// most 2^28 voxels (each TR stores its echo once, at a 32-bit byte offset
-// from the TR's row).  max_angle: the wave's fisp_table_max_angle.
+// polynomial; q0: fl(h 2/pi) <= 1/2, every reduction index is 0; plain: one
+// slice profile, one repetition, no undersampling and at most 2^28 voxels
+// (each TR stores its echo once, at a 32-bit byte offset from the TR's row);
+// simple: plain without the direct echo.  max_angle: the launch's largest flip
+// angle, from the end of its RF table.
 struct FispWaveForm {
-    bool wide, simple, q0, direct_echo;
+    bool wide, plain, simple, q0, direct_echo;
 };
 
-__device__ inline FispWaveForm fisp_wave_form(const FispArgs& a, int voxel, float max_angle) {
+__device__ inline FispWaveForm fisp_wave_form(const FispArgs& a, int voxel) {
     FispWaveForm f;
+    const float max_angle = a.table[a.nslices * a.nTR].x;
     const float h = 0.5f * (max_angle * fabsf(a.tissue.B1(voxel)));
     f.direct_echo = fisp_direct_echo(a, a.tissue.T2(voxel), a.tissue.B0(voxel));
     f.wide = __any(!(h <= 64.0f));
     f.q0 = !__any(!(h * 0.63661977236758134f <= 0.5f));
-    f.simple = !f.direct_echo && a.nslices == 1 && a.repetitions == 1 && a.usf == 1 && a.tissue.nvoxels <= (1 << 28);
+    f.plain = a.nslices == 1 && a.repetitions == 1 && a.usf == 1 && a.tissue.nvoxels <= (1 << 28);
+    f.simple = f.plain && !f.direct_echo;
     return f;
 }
 

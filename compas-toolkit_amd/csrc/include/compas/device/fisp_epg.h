@@ -243,8 +243,8 @@ __device__ __forceinline__ void fisp_epg_voxel_form(const FispArgs& a, int voxel
 // fisp_epg_voxel_form in the form the wave needs (fisp_wave_form), decided
 // once per wave so that the TR loop carries no test for it.
 template<int SPL, int LPV>
-__device__ __forceinline__ void fisp_epg_voxel(const FispArgs& a, int voxel, int sub, float max_angle) {
-    const FispWaveForm f = fisp_wave_form(a, voxel, max_angle);
+__device__ __forceinline__ void fisp_epg_voxel(const FispArgs& a, int voxel, int sub) {
+    const FispWaveForm f = fisp_wave_form(a, voxel);
     if (f.wide) {
         fisp_epg_voxel_form<SPL, LPV, HALF_WIDE, false>(a, voxel, sub, f.direct_echo);
     } else if (!f.simple) {

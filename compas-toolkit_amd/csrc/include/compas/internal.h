@@ -10,6 +10,7 @@ namespace compas {
 
 namespace kernels {
 struct FispArgs;
+struct FispPlanes;
 struct PssfpArgs;
 struct PssfpTableJob;
 struct PssfpMapArgs;
@@ -103,8 +104,15 @@ bool spiral_sum_mfma(
     const CompasContext& ctx, const TissueParameters& p, const cfloat* A, const cfloat* Ab, const cfloat* coils,
     int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out);
 
-// Per (slice, TR) RF table of the FISP kernels: (deg2rad |RF|, cos phi, sin phi, 0).
+// Per (slice, TR) RF table of the FISP kernels (FispArgs::table).
 Array<float4, 1> fisp_rf_table(const CompasContext& ctx, const FISPSequence& seq);
+
+// The recursion of a train of real pulses and the planes of one pass of its
+// tangents (fisp_real.hip; `mask`: TangentSet); does nothing for other trains.
+void launch_fisp_real(const CompasContext& ctx, const kernels::FispArgs& a, int mask, const kernels::FispPlanes& out);
+void launch_fisp_real_tangents(
+    const CompasContext& ctx, const kernels::FispArgs& a, int mask, const kernels::FispPlanes& out);
+int simd_count(int device);
 
 // simulate_magnetization(FISP) into the caller's device buffer `echos`
 // ([nTR * usf][nvoxels], `capacity` complex values) without allocating: the

@@ -30,40 +30,56 @@
 #include "compas/device/common.h"
 #include "compas/device/fisp_common.h"
 #include "compas/device/fisp_epg.h"
+#include "compas/device/fisp_real.h"
 #include "compas/internal.h"
 
 namespace compas {
 namespace kernels {
 
-// table[i] for i < nslices nTR, then a zero entry at nslices nTR (the
-// recursion loads the entry of the TR after its last one); nslices nTR + 1
-// threads.
-__global__ void fisp_rf_table(const cfloat* RF, const cfloat* profiles, int nTR, int nslices, float4* table) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > nTR * nslices) return;
-    if (i == nTR * nslices) {
-        table[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        return;
+// The RF table (FispArgs::table) with its two closing entries.  One workgroup
+// of 1024 threads: every wave of the recursion needs the train's largest flip
+// angle and whether its pulses are real, and would otherwise look through the
+// whole table for them.
+__global__ void __launch_bounds__(1024) fisp_rf_table(
+    const cfloat* RF, const cfloat* profiles, int nTR, int nslices, float4* table) {
+    __shared__ float s_max[16];
+    __shared__ int s_real;
+    const int total = nTR * nslices;
+    if (threadIdx.x == 0) s_real = 1;
+    __syncthreads();
+    float largest = 0.0f;
+    bool real = true;
+    for (int i = threadIdx.x; i < total; i += 1024) {
+        const cfloat p = profiles[i], r = RF[i % nTR];
+        const cfloat rf = {p.re * r.re - p.im * r.im, p.re * r.im + p.im * r.re};
+        const float a = hypotf(rf.re, rf.im);
+        float c = 1.0f, s = 0.0f;
+        if (a > FLT_MIN) {  // epg.cuh:64-67
+            c = rf.re / a;
+            s = rf.im / a;
+        }
+        table[i] = make_float4(dev::DEG2RAD_F * a, c, s, 0.0f);
+        largest = fmaxf(largest, dev::DEG2RAD_F * a);
+        real = real && s == 0.0f;
     }
-    int n = i % nTR;
-    cfloat p = profiles[i], r = RF[n];
-    cfloat rf = {p.re * r.re - p.im * r.im, p.re * r.im + p.im * r.re};
-    float a = hypotf(rf.re, rf.im);
-    float c = 1.0f, s = 0.0f;
-    if (a > FLT_MIN) {  // epg.cuh:64-67
-        c = rf.re / a;
-        s = rf.im / a;
+    for (int off = 32; off > 0; off >>= 1) largest = fmaxf(largest, __shfl_xor(largest, off));
+    if (threadIdx.x % 64 == 0) s_max[threadIdx.x / 64] = largest;
+    if (!real) s_real = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) largest = fmaxf(largest, s_max[w]);
+        table[total] = make_float4(largest, 0.0f, 0.0f, s_real ? 1.0f : 0.0f);
+        table[total + 1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
-    table[i] = make_float4(dev::DEG2RAD_F * a, c, s, 0.0f);
 }
 
 template<int SPL, int LPV>
 __global__ void __launch_bounds__(64) fisp_epg(FispArgs a) {
     const int sub = (LPV > 1) ? int(threadIdx.x % LPV) : 0;
     const int voxel = (blockIdx.x * 64 + threadIdx.x) / LPV;
-    const float max_angle = fisp_table_max_angle(a);  // while every lane is active
+    if (fisp_real_train(a)) return;  // fisp_real runs instead
     if (voxel >= a.tissue.nvoxels) return;  // whole LPV groups leave together
-    fisp_epg_voxel<SPL, LPV>(a, voxel, sub, max_angle);
+    fisp_epg_voxel<SPL, LPV>(a, voxel, sub);
 }
 
 }  // namespace kernels
@@ -160,16 +176,15 @@ static FispLauncher fisp_launcher_lpv4(int spl) {
 
 Array<float4, 1> fisp_rf_table(const CompasContext& ctx, const FISPSequence& seq) {
     const int nTR = int(seq.RF_train.size(0)), nslices = int(seq.sliceprofiles.size(0));
-    auto table = ctx.empty<float4, 1>({int64_t(nslices) * nTR + 1});
+    auto table = ctx.empty<float4, 1>({int64_t(nslices) * nTR + 2});
     KernelScope ks(ctx, "fisp_rf_table");
-    const int total = nslices * nTR + 1;
-    kernels::fisp_rf_table<<<dev::div_ceil(total, 256), 256, 0, ctx.stream()>>>(
+    kernels::fisp_rf_table<<<1, 1024, 0, ctx.stream()>>>(
         seq.RF_train.data(), seq.sliceprofiles.data(), nTR, nslices, table.data());
     check_launch("fisp_rf_table");
     return table;
 }
 
-static int simd_count(int device) {
+int simd_count(int device) {
     static int cached[64] = {0};
     if (device >= 0 && device < 64 && cached[device]) return cached[device];
     hipDeviceProp_t prop;
@@ -265,7 +280,7 @@ Array<cfloat, 2> simulate_magnetization(
 
 static constexpr int64_t kRfTableScratchEntries = int64_t(1) << 16;  // (slice, TR) pairs: 1 MiB
 
-static __device__ __align__(256) float4 scratch[kRfTableScratchEntries + 1];  // and the terminating zero entry
+static __device__ __align__(256) float4 scratch[kRfTableScratchEntries + 2];  // and the two closing entries
 
 static float4* scratch_address(int device) {
     static std::mutex mutex;
@@ -309,8 +324,7 @@ void simulate_magnetization_into(
         return;
     }
     float4* table = scratch_address(ctx.device());
-    const int total = int(nslices * nTR) + 1;
-    kernels::fisp_rf_table<<<dev::div_ceil(total, 256), 256, 0, ctx.stream()>>>(
+    kernels::fisp_rf_table<<<1, 1024, 0, ctx.stream()>>>(
         seq.RF_train.data(), seq.sliceprofiles.data(), int(nTR), int(nslices), table);
     check_launch("fisp_rf_table");
     launch_fisp_epg(ctx, parameters, seq, table, echos, false);
@@ -352,13 +366,18 @@ static void launch_fisp_epg(
     FispLauncher fn = lpv == 1 ? fisp_launcher_lpv1(spl) : lpv == 2 ? fisp_launcher_lpv2(spl) : fisp_launcher_lpv4(spl);
     COMPAS_CHECK(fn != nullptr);
     unsigned blocks = dev::div_ceil(int64_t(nv) * lpv, 64);
+    // both forms are launched, and the one that does not suit the train leaves
+    // at once: what the train is like is known on the device only
+    const auto launch = [&] {
+        launch_fisp_real(ctx, a, kernels::TM_ECHO, kernels::FispPlanes {{echos}});
+        fn(a, blocks, ctx.stream());
+        check_launch("fisp_epg");
+    };
     if (timed) {
         KernelScope ks(ctx, "fisp_epg");
-        fn(a, blocks, ctx.stream());
-        check_launch("fisp_epg");
+        launch();
     } else {
-        fn(a, blocks, ctx.stream());
-        check_launch("fisp_epg");
+        launch();
     }
 }
 

@@ -1,10 +1,11 @@
 // Work-table launch of the FISP recursion for the request server: one
 // launch runs voxel blocks of several simulations (of different requests,
 // voxel counts and sequences) that share the state count.  See
-// compas/device/fisp_epg.h for the recursion and fisp.hip for the per-call
-// launch; a voxel's arithmetic is the same in both with one lane per voxel.
+// compas/device/fisp_epg.h and fisp_real.h for the recursion and fisp.hip and
+// fisp_real.hip for the per-call launches.
 
 #include "compas/device/fisp_epg.h"
+#include "compas/device/fisp_real.h"
 #include "compas/internal.h"
 
 namespace compas {
@@ -17,9 +18,12 @@ __global__ void __launch_bounds__(64) fisp_epg_table(const FispArgs* __restrict_
     const int2 it = items[blockIdx.x];
     const FispArgs a = jobs[it.x];
     const int voxel = it.y * 64 + int(threadIdx.x);
-    const float max_angle = fisp_table_max_angle(a);  // while every lane is active
     if (voxel >= a.tissue.nvoxels) return;
-    fisp_epg_voxel<SPL, 1>(a, voxel, 0, max_angle);
+    if (fisp_real_train(a)) {
+        fisp_real_voxel<SPL, 1, TM_ECHO>(a, FispPlanes {{a.echos}}, voxel, 0);
+    } else {
+        fisp_epg_voxel<SPL, 1>(a, voxel, 0);
+    }
 }
 
 }  // namespace kernels

@@ -36,6 +36,7 @@
 
 #include "compas/device/common.h"
 #include "compas/device/fisp_common.h"
+#include "compas/device/fisp_real.h"
 #include "compas/device/tangent_set.h"
 #include "compas/internal.h"
 
@@ -46,10 +47,6 @@ namespace kernels {
 __device__ inline cfloat times_i(cfloat z) {
     return {-z.im, z.re};
 }
-
-struct FispPlanes {
-    cfloat* p[5];  // [nTR * usf][nvoxels] each, in the order of TangentSet
-};
 
 // The three rows of a 3x3 real matrix applied to an EPG state (F+, F-, Z)
 // in the (S = F+ + F-, D = F+ - F-) form the recursion uses: rows 0/1 act on
@@ -367,9 +364,9 @@ template<int SPL, int LPV, int MASK>
 __global__ void __launch_bounds__(64) fisp_epg_tangents(FispArgs a, FispPlanes out) {
     const int sub = (LPV > 1) ? int(threadIdx.x % LPV) : 0;
     const int voxel = (blockIdx.x * 64 + threadIdx.x) / LPV;
-    const float max_angle = fisp_table_max_angle(a);  // while every lane is active
+    if (fisp_real_train(a)) return;  // fisp_real_tangents runs instead
     if (voxel >= a.tissue.nvoxels) return;  // whole LPV groups leave together
-    const FispWaveForm f = fisp_wave_form(a, voxel, max_angle);
+    const FispWaveForm f = fisp_wave_form(a, voxel);
     if (f.wide) {
         fisp_tangents_voxel<SPL, LPV, MASK, HALF_WIDE, false>(a, out, voxel, sub, f.direct_echo);
     } else if (!f.simple) {
@@ -559,6 +556,7 @@ std::vector<Array<cfloat, 2>> simulate_magnetization_tangents(
         const int lpv = lanes_per_voxel(seq.max_state, spl);
         launcher_for_mask(pass, lpv, &fn, &spl);
         KernelScope ks(ctx, "fisp_epg_tangents");
+        launch_fisp_real(ctx, a, pass, o);
         fn(a, o, unsigned(dev::div_ceil(int64_t(nv) * lpv, 64)), ctx.stream());
         check_launch("fisp_epg_tangents");
     }
