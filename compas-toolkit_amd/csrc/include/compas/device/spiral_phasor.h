@@ -1,0 +1,39 @@
+#pragma once
+// Per-voxel constants and phasors of the spiral sample factor
+//   E_rv^s = exp(s (-dt / T2_v + i (dk_r . x_v + 2 pi dt B0_v)))
+// (spiral_view.cuh:59-73) shared by the two-level spiral kernels.
+
+#include "compas/device/common.h"
+
+namespace compas {
+namespace kernels {
+
+// One voxel: x, y, dt B0 in turns, and the decay exponent per sample, base 2
+struct alignas(16) SpiralVoxel {
+    double turns;
+    float x, y;
+    float decay;
+    float T2;
+    float pad[2];
+};
+
+__global__ void spiral_voxels(dev::TissueView t, float dt, SpiralVoxel* __restrict__ out);
+
+// Turns per sample of a voxel; dkx, dky: delta_k / 2 pi
+__device__ __forceinline__ double spiral_turns(const SpiralVoxel& v, double dkx, double dky) {
+    return fma(dkx, double(v.x), fma(dky, double(v.y), v.turns));
+}
+
+// 2^(log2_mag) e^{2 pi i turns}: the phase is reduced to half a turn in FP64.
+// The hardware's sine and cosine of a phase in turns are within 1.3e-7 there
+// (measured over [-1/2, 1/2], RMS 3.5e-8: no worse than the polynomials of
+// sincos_reduced at a third of the instructions), its base-2 exponential
+// within 8.3e-8 relative.
+__device__ __forceinline__ cfloat spiral_phasor(float log2_mag, double turns) {
+    const float f = float(turns - rint(turns));
+    const float m = __builtin_amdgcn_exp2f(log2_mag);
+    return {m * __builtin_amdgcn_cosf(f), m * __builtin_amdgcn_sinf(f)};
+}
+
+}  // namespace kernels
+}  // namespace compas

@@ -1,31 +1,40 @@
 // Spiral sums out[c][r][s] = sum_v C[c][v] (A[r][v] + (s - ns/2) Ab[r][v]) E_rv^s
-// (signal: A only; J.v: both amplitudes) with the voxel sum on MFMA.
+// (signal: A only; J.v: both amplitudes) with the voxel sum on MFMA (BF16 hi +
+// lo, or hi only; FP32 accumulation).
 //
-// Per readout this is a complex GEMM, rows (coil, amplitude) x K = voxels x
-// N = samples, whose B operand E_rv^s is generated: E^s is a geometric
-// sequence in s for each voxel, so a lane that keeps its voxels fixed and walks
-// the samples needs one complex multiply per element.  Hence the loop order:
-// a wave owns one readout, a range of voxels and a block of up to 512 samples,
-// and keeps the accumulators of all 32 sixteen-sample tiles (4 floats per
-// lane each) while it walks its voxels 16 at a time (one K step of
-// v_mfma_f32_16x16x32_bf16).  Per K step each lane evaluates, for its four
-// voxels, E^(s0 + n) from an FP64 phase and E^16 (the tile step) once, then
-// per tile: four complex multiplies, the BF16 hi + lo split of four pairs and
-// three MFMAs (hi*hi, hi*lo, lo*hi; one with the single-product precision).
+// With s = sb + S t + n, S = 32 CT, E^s = E^(sb + S t) E^n, so a readout's sum
+// is a complex GEMM with rows (coil, t), columns n < S and K = voxels: A = C A_r
+// E^(sb + S t), B = E^n.  Per voxel and readout nc T + S elements are generated
+// instead of one for every sample (96 instead of 512 at 4 coils x 512
+// samples), for the same MFMA products.  Of the two amplitudes, (s - ns/2) Ab =
+// (sb + S t - ns/2) Ab + n Ab: the first term joins A's rows, the second has
+// rows of its own, whose sum the epilogue multiplies by n.
 //
-// Rows of the 16-row A operand (lane group g = l / 16 receives result rows
-// 4 g .. 4 g + 3 of its column):
-//   J.v    row 4 c + (Re Wa, Im Wa, Re Wb, Im Wb), four coils per group; the
-//          two amplitude sums are stored as separate planes and the
-//          reduction forms Wa-sum + (s - ns/2) Wb-sum;
-//   signal row 2 c + (Re W, Im W), eight coils per group.
-// W = C A (or C Ab) as (w_re, -w_im) / (w_im, w_re) pairs along the
-// interleaved K.  Voxel ranges of one readout are summed by a second pass
-// over the partial planes in FP64 (deterministic).
+// A wave owns a readout and a voxel range and walks it eight voxels at a time
+// (one K step of v_mfma_f32_32x32x16_bf16):
+//   * generate: lane (voxel l % 8, slot q = l / 8) forms E^q and E^(sb + S q),
+//     one phasor each, steps through E^(q + 8 m) with E^8 = (E^4)^2 from a
+//     neighbouring lane, splits them and leaves B's hi and lo words and A_r
+//     E^(sb + S q) in LDS;
+//   * contract: lane l reads B's column l % 32 and, for its row (coil, t), four
+//     voxels' amplitudes, multiplies them with the coil map, and splits the rows
+//     of the real and of the imaginary part, (w_re, -w_im) and (w_im, w_re).
+// Rows: T is a power of two up to 8, row = coil T + t, 32 to a tile, RT tiles
+// (coils beyond nc and samples beyond ns are computed and not stored); 32 RT CT
+// accumulator registers.  Voxel ranges of one readout are summed by a second
+// pass over the partial planes in FP64 (deterministic).
 //
-// Layout of v_mfma_f32_16x16x32_bf16 (wave64): lane l supplies row (A) or
-// column (B) l % 16 and K elements 8 (l / 16) .. + 7; result element j of lane
-// l is row 4 (l / 16) + j, column l % 16.
+// What bounds it: VALU issue (the splits are a third of it) at the clock that
+// the matrix units leave.  At 4 coils x 1120 x 512 over 50176 voxels the signal
+// takes 4.1 ms and J.v 6.8 ms with their amplitude passes (13.1 and 13.8 ms
+// when every sample's element was generated), VALU busy 74% and MFMA 35% of the
+// cycles at 1.8 GHz.  Tried without gain: the next step's generation beside the
+// MFMAs (two LDS buffers, with and without scheduling groups), the two
+// amplitudes in two waves of a workgroup, four waves per SIMD.
+//
+// Layout of v_mfma_f32_32x32x16_bf16 (wave64): lane l supplies row (A) or
+// column (B) l % 32 and K elements 8 (l / 32) .. + 7; result element e of lane l
+// is row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32.
 
 #include <algorithm>
 #include <cstdint>
@@ -33,156 +42,192 @@
 
 #include "compas/device/common.h"
 #include "compas/device/mfma_tile.h"
+#include "compas/device/spiral_phasor.h"
 #include "compas/internal.h"
 
 namespace compas {
 namespace kernels {
-
-typedef float f32x4s __attribute__((ext_vector_type(4)));
-
 
 __device__ inline mfma::bf16x8 pack_bf16x8(const uint32_t (&w)[4]) {
     const uint4 v = {w[0], w[1], w[2], w[3]};
     return __builtin_bit_cast(mfma::bf16x8, v);
 }
 
-// partial[split][c][r][s] over voxels [v_begin, v_end) of split blockIdx.y;
-// grid (nr, splits, sample passes), block 64.  FULL: every pass holds
-// SSM_TILES whole tiles (ns a multiple of 16 SSM_TILES), so the tile loop
-// carries no test.
-template<bool TWO, bool LO, int SSM_TILES, bool FULL>
-__global__ void __launch_bounds__(64) spiral_sum_mfma(
-    dev::TissueView tissue, const cfloat* __restrict__ A, const cfloat* __restrict__ Ab,
-    const cfloat* __restrict__ coils, int nc, const cfloat* __restrict__ delta_k, int nr, int ns, float dt,
-    int v_chunk, cfloat* __restrict__ partial) {
-    constexpr int P = LO ? mfma::P_BF16X3 : mfma::P_BF16X1;
-    const int lane = threadIdx.x;
-    const int n = lane & 15, g = lane >> 4;
-    const int r = blockIdx.x;
-    const int nv = tissue.nvoxels;
-    const int v_begin = blockIdx.y * v_chunk, v_end = min(nv, v_begin + v_chunk);
-    const int sb = blockIdx.z * 16 * SSM_TILES;  // first sample of the pass
-    const int ntiles = min(SSM_TILES, (ns - sb + 15) / 16);
-    const size_t row = size_t(r) * nv;
-    const cfloat dk = delta_k[r];
-    const double two_pi_dt = double(dt) * dev::TWO_PI;
-
-    // A-operand row of this lane
-    const int arow = n;
-    const int acoil = TWO ? (arow >> 2) : (arow >> 1);
-    const bool a_im = TWO ? (arow & 1) : (arow & 1);
-    const bool a_b = TWO && (arow & 2);  // row of the second amplitude
-    const bool a_ok = acoil < nc;
-
-    f32x4s acc[SSM_TILES];
-#pragma unroll
-    for (int t = 0; t < SSM_TILES; t++) acc[t] = f32x4s {0.0f, 0.0f, 0.0f, 0.0f};
-
-    const int s_lane = sb + n;  // the lane's sample in tile 0
-    for (int vk = v_begin; vk < v_end; vk += 16) {
-        // the lane's four voxels of this K step (K elements 8 g .. 8 g + 7).
-        // Their phase slope, decay and 16-sample step do not depend on the
-        // lane's sample: lane n of the group evaluates them for voxel n % 4,
-        // and the group's lanes read them from there
-        double theta_own;
-        float decay_own;
-        cfloat st16_own;
-        {
-            const int v = vk + 4 * g + (n & 3);
-            const int vv = v < v_end ? v : v_begin;
-            const float R2 = 1.0f / tissue.T2(vv);
-            theta_own = double(dk.re) * double(tissue.x(vv)) + double(dk.im) * double(tissue.y(vv)) +
-                two_pi_dt * double(tissue.B0(vv));
-            decay_own = -dt * R2;
-            st16_own = dev::polar_reduced(expf(16.0f * decay_own), 16.0 * theta_own);
-        }
-        cfloat ph[4], st16[4];
-        uint32_t ahw[4], alw[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int v = vk + 4 * g + j;
-            const bool ok = v < v_end;
-            const int src = (lane & ~15) | j;
-            const double theta = __shfl(theta_own, src);
-            const float decay = __shfl(decay_own, src);
-            st16[j] = {__shfl(st16_own.re, src), __shfl(st16_own.im, src)};
-            ph[j] = ok ? dev::polar_reduced(expf(float(s_lane) * decay), double(s_lane) * theta) : cfloat {0, 0};
-            // A: W = C[coil][v] (A or Ab)[r][v] as a (re, -im) or (im, re) pair
-            cfloat w = {0.0f, 0.0f};
-            if (a_ok && ok) w = dev::cmul(coils[size_t(acoil) * nv + v], a_b ? Ab[row + v] : A[row + v]);
-            const float e0 = a_im ? w.im : w.re;
-            const float e1 = a_im ? w.re : -w.im;
-            mfma::split_pair<P>(e0, e1, ahw[j], alw[j]);
-        }
-        const mfma::bf16x8 ahi = pack_bf16x8(ahw);
-        const mfma::bf16x8 alo = pack_bf16x8(alw);
-#pragma unroll
-        for (int t = 0; t < SSM_TILES; t++) {
-            if (FULL || t < ntiles) {
-                uint32_t bhw[4], blw[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) mfma::split_pair<P>(ph[j].re, ph[j].im, bhw[j], blw[j]);
-                const mfma::bf16x8 bhi = pack_bf16x8(bhw);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi, bhi, acc[t], 0, 0, 0);
-                if constexpr (LO) {
-                    const mfma::bf16x8 blo = pack_bf16x8(blw);
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi, blo, acc[t], 0, 0, 0);
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo, bhi, acc[t], 0, 0, 0);
-                }
-#pragma unroll
-                for (int j = 0; j < 4; j++) ph[j] = dev::cmul(ph[j], st16[j]);
-            }
-        }
-    }
-
-    // result rows 4 g + j of column n (sample sb + 16 t + n); with two
-    // amplitudes the second one goes to its own plane (the reduction applies
-    // the (s - ns/2) factor), so the accumulators are only stored here
-    const size_t plane = size_t(nc) * nr * ns;
-    cfloat* base = partial + size_t(blockIdx.y) * (TWO ? 2 : 1) * plane;
-#pragma unroll
-    for (int t = 0; t < SSM_TILES; t++) {
-        const int s = sb + 16 * t + n;
-        if (FULL || (t < ntiles && s < ns)) {
-            if constexpr (TWO) {
-                const int c = g;
-                if (c < nc) {
-                    const size_t o = (size_t(c) * nr + r) * ns + s;
-                    base[o] = {acc[t][0], acc[t][1]};
-                    base[plane + o] = {acc[t][2], acc[t][3]};
-                }
-            } else {
-                const int c0 = 2 * g;
-                if (c0 < nc) base[(size_t(c0) * nr + r) * ns + s] = {acc[t][0], acc[t][1]};
-                if (c0 + 1 < nc) base[(size_t(c0 + 1) * nr + r) * ns + s] = {acc[t][2], acc[t][3]};
-            }
-        }
+// The pairs of w in the rows of the real and of the imaginary part, (w_re,
+// -w_im) and (w_im, w_re), split into BF16 hi + lo: the conversions take the
+// sign and the order for nothing.
+template<bool LO>
+__device__ __forceinline__ void split_rows(cfloat w, uint32_t& rh, uint32_t& rl, uint32_t& ih, uint32_t& il) {
+    const mfma::bf16x2 h = {(__bf16)w.re, (__bf16)-w.im}, hi = {(__bf16)w.im, (__bf16)w.re};
+    rh = __builtin_bit_cast(uint32_t, h);
+    ih = __builtin_bit_cast(uint32_t, hi);
+    if constexpr (LO) {
+        const float re = w.re - __builtin_bit_cast(float, rh << 16), im = w.im - __builtin_bit_cast(float, ih << 16);
+        rl = __builtin_bit_cast(uint32_t, mfma::bf16x2 {(__bf16)re, (__bf16)-im});
+        il = __builtin_bit_cast(uint32_t, mfma::bf16x2 {(__bf16)im, (__bf16)re});
+    } else {
+        rl = il = 0u;
     }
 }
 
-// out[i] = sum over the splits (FP64, in order); with two amplitudes each
-// split holds the plane of the first and then of the second, and
-// out = first + (s - ns/2) second, s = i % ns
-template<bool TWO>
-__global__ void spiral_sum_reduce(
-    const cfloat* __restrict__ partial, int splits, int64_t n, int ns, cfloat* __restrict__ out) {
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
-        double re = 0.0, im = 0.0, bre = 0.0, bim = 0.0;
-        for (int k = 0; k < splits; k++) {
-            const size_t o = size_t(k) * (TWO ? 2 : 1) * size_t(n) + size_t(i);
-            const cfloat p = partial[o];
-            re += p.re;
-            im += p.im;
-            if constexpr (TWO) {
-                const cfloat q = partial[o + size_t(n)];
-                bre += q.re;
-                bim += q.im;
+__global__ void spiral_voxels(dev::TissueView t, float dt, SpiralVoxel* __restrict__ out) {
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= t.nvoxels) return;
+    SpiralVoxel o {};
+    o.turns = double(dt) * double(t.B0(v));
+    o.x = t.x(v);
+    o.y = t.y(v);
+    o.T2 = t.T2(v);
+    o.decay = float(-1.4426950408889634 * double(dt) / double(o.T2));  // log2(e)
+    out[v] = o;
+}
+
+// grid (nr, voxel ranges, sample passes), block 64
+typedef float f32x16s __attribute__((ext_vector_type(16)));
+
+template<int CT, int RT, bool TWO, bool LO>
+__global__ void __launch_bounds__(64, 2) spiral_sum_split(
+    const SpiralVoxel* __restrict__ voxels, int nv, const cfloat* __restrict__ A, const cfloat* __restrict__ Ab,
+    const cfloat* __restrict__ coils, int nc, const cfloat* __restrict__ delta_k, int nr, int ns, int tbits,
+    int v_chunk, cfloat* __restrict__ partial) {
+    static_assert(!TWO || RT == 2, "the two amplitudes take a row tile each");
+    constexpr int P = LO ? mfma::P_BF16X3 : mfma::P_BF16X1;
+    constexpr int S = 32 * CT;
+    __shared__ __align__(16) uint32_t b_hi[S * 8], b_lo[LO ? S * 8 : 4];
+    __shared__ __align__(16) float2 amp[TWO ? 2 : 1][8 * 8];
+    const int lane = threadIdx.x;
+    const int gv = lane & 7, q = lane >> 3;      // generating: voxel of the step, slot
+    const int col = lane & 31, half = lane >> 5;  // contracting: row / column, half of the voxels
+    const int r = blockIdx.x;
+    const int v_begin = blockIdx.y * v_chunk, v_end = min(nv, v_begin + v_chunk);
+    const int sb = blockIdx.z * (S << tbits);
+    const int t = col & ((1 << tbits) - 1);
+    const size_t row = size_t(r) * nv;
+    const cfloat dk = delta_k[r];
+    const double dkx = double(dk.re) / dev::TWO_PI, dky = double(dk.im) / dev::TWO_PI;
+    const cfloat* coil_row[TWO ? 1 : RT];
+#pragma unroll
+    for (int i = 0; i < (TWO ? 1 : RT); i++) {
+        const int c = (col >> tbits) + i * (32 >> tbits);
+        coil_row[i] = coils + size_t(min(c, nc - 1)) * nv;
+    }
+
+    f32x16s acc[RT][2][CT];
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[i][k][j][e] = 0.0f;
+
+    const float s_amp = float(sb + S * q);  // the slot's sample
+    const float tau = s_amp - 0.5f * float(ns);
+    // the next step's voxel is loaded a step ahead
+    SpiralVoxel nx;
+    cfloat na, nb {};
+    auto load = [&](int vk) {
+        const int v = min(vk + gv, v_end - 1);
+        nx = voxels[v];
+        na = A[row + v];
+        if constexpr (TWO) nb = Ab[row + v];
+        if (vk + gv >= v_end) na = nb = {0.0f, 0.0f};
+    };
+    load(v_begin);
+    for (int vk = v_begin; vk < v_end; vk += 8) {
+        const SpiralVoxel x = nx;
+        const cfloat a = na, ab = nb;
+        load(vk + 8);
+        cfloat cm[TWO ? 1 : RT][4];
+#pragma unroll
+        for (int i = 0; i < (TWO ? 1 : RT); i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) cm[i][j] = coil_row[i][min(vk + 4 * half + j, nv - 1)];
+
+        const double turns = spiral_turns(x, dkx, dky);
+        cfloat ph = spiral_phasor(float(q) * x.decay, double(q) * turns);
+        cfloat e8 = {__shfl(ph.re, 32 + gv), __shfl(ph.im, 32 + gv)};
+        e8 = dev::cmul(e8, e8);
+        const cfloat w = spiral_phasor(s_amp * x.decay, double(s_amp) * turns);
+        if constexpr (TWO) {
+            const cfloat u = dev::cmul(cfloat {fmaf(tau, ab.re, a.re), fmaf(tau, ab.im, a.im)}, w);
+            const cfloat ub = dev::cmul(ab, w);
+            amp[0][lane] = make_float2(u.re, u.im);
+            amp[1][lane] = make_float2(ub.re, ub.im);
+        } else {
+            const cfloat u = dev::cmul(a, w);
+            amp[0][lane] = make_float2(u.re, u.im);
+        }
+#pragma unroll
+        for (int m = 0; m < S / 8; m++) {
+            uint32_t h, l;
+            mfma::split_pair<P>(ph.re, ph.im, h, l);
+            b_hi[64 * m + lane] = h;
+            if constexpr (LO) b_lo[64 * m + lane] = l;
+            if (m + 1 < S / 8) ph = dev::cmul(ph, e8);
+        }
+        __syncthreads();  // one wave: orders the LDS accesses
+
+        mfma::bf16x8 bh[CT], bl[CT];
+#pragma unroll
+        for (int j = 0; j < CT; j++) {
+            bh[j] = *reinterpret_cast<const mfma::bf16x8*>(&b_hi[(32 * j + col) * 8 + 4 * half]);
+            if constexpr (LO) bl[j] = *reinterpret_cast<const mfma::bf16x8*>(&b_lo[(32 * j + col) * 8 + 4 * half]);
+        }
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+            uint32_t rh[4], rl[4], ih[4], il[4];
+            const float4* p = reinterpret_cast<const float4*>(&amp[TWO ? i : 0][8 * t + 4 * half]);
+            const float4 p01 = p[0], p23 = p[1];
+            const cfloat pv[4] = {{p01.x, p01.y}, {p01.z, p01.w}, {p23.x, p23.y}, {p23.z, p23.w}};
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                split_rows<LO>(dev::cmul(cm[TWO ? 0 : i][j], pv[j]), rh[j], rl[j], ih[j], il[j]);
+            const mfma::bf16x8 ah[2] = {pack_bf16x8(rh), pack_bf16x8(ih)}, al[2] = {pack_bf16x8(rl), pack_bf16x8(il)};
+            // one product over all tiles, then the next: no MFMA waits for the one before it
+#pragma unroll
+            for (int product = 0; product < (LO ? 3 : 1); product++)
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+#pragma unroll
+                    for (int j = 0; j < CT; j++)
+                        acc[i][k][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            product == 2 ? al[k] : ah[k], product == 1 ? bl[j] : bh[j], acc[i][k][j], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+
+    cfloat* base = partial + size_t(blockIdx.y) * (size_t(nc) * nr * ns);
+#pragma unroll
+    for (int i = 0; i < (TWO ? 1 : RT); i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            const int rho = 32 * i + 8 * (e / 4) + 4 * half + (e % 4);
+            const int c = rho >> tbits, tt = rho & ((1 << tbits) - 1);
+#pragma unroll
+            for (int j = 0; j < CT; j++) {
+                const int n = 32 * j + col, s = sb + S * tt + n;
+                if (c < nc && s < ns) {
+                    cfloat o = {acc[i][0][j][e], acc[i][1][j][e]};
+                    if constexpr (TWO) {
+                        o.re = fmaf(float(n), acc[RT - 1][0][j][e], o.re);
+                        o.im = fmaf(float(n), acc[RT - 1][1][j][e], o.im);
+                    }
+                    base[(size_t(c) * nr + r) * ns + s] = o;
+                }
             }
         }
-        if constexpr (TWO) {
-            const double sp = double(i % ns) - 0.5 * double(ns);
-            re = fma(sp, bre, re);
-            im = fma(sp, bim, im);
+}
+
+// out[i] = sum over the splits (FP64, in order)
+__global__ void spiral_sum_reduce(const cfloat* __restrict__ partial, int splits, int64_t n, cfloat* __restrict__ out) {
+    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
+        double re = 0.0, im = 0.0;
+        for (int k = 0; k < splits; k++) {
+            const cfloat p = partial[size_t(k) * size_t(n) + size_t(i)];
+            re += p.re;
+            im += p.im;
         }
         out[i] = {float(re), float(im)};
     }
@@ -195,56 +240,57 @@ bool spiral_sum_mfma(
     int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out) {
     if (precision == ContractionPrecision::FP32) return false;
     const bool two = Ab != nullptr;
-    if (nc > (two ? 4 : 8)) return false;  // one 16-row group; more coils: the VALU form
+    if (nc > (two ? 4 : 8)) return false;  // more coils than the row tiles hold: the VALU form
     const bool lo = precision == ContractionPrecision::BF16x3 || precision == ContractionPrecision::FP16x3;
     const int nr = t.nreadouts, ns = t.samples_per_readout, nv = p.nvoxels;
-    // sample block per pass: 32 tiles of 16 samples (128 accumulator
-    // registers, two waves per SIMD).  Measured at 4 coils x 1120 x 512 over
-    // 50176 voxels: 16.5 ms per launch, against 18.7 ms with 16 tiles (four
-    // waves per SIMD but twice the per-voxel set-up per sample).
-    constexpr int tiles = 32;
-    const int passes = int(dev::div_ceil(ns, 16 * tiles));
-    // voxel splits so that the grid holds about four waves per SIMD
-    const int want = int(std::max<int64_t>(1, dev::div_ceil(4 * 1024, int64_t(nr) * passes)));
-    const int max_splits = int(dev::div_ceil(nv, 16));
-    const int splits0 = std::min(want, max_splits);
-    const int v_chunk = int(dev::div_ceil(dev::div_ceil(nv, splits0), 16)) * 16;
+    // S = 64 columns for more than 256 samples (half as many rows to generate per
+    // column), 32 below; up to 8 S samples a pass
+    const int ct = ns > 256 ? 2 : 1;
+    const int S = 32 * ct;
+    int tbits = 0;
+    while (tbits < 3 && (S << tbits) < ns) tbits++;
+    const int passes = int(dev::div_ceil(ns, S << tbits));
+    const int rt = two || (nc << tbits) > 32 ? 2 : 1;
+    // voxel splits: about eight waves per SIMD in the grid (two or three are
+    // resident; with four, 1.4 rounds of them took 10% longer), sixteen K steps
+    // each at least
+    const int want = int(std::max<int64_t>(1, dev::div_ceil(8 * 1024, int64_t(nr) * passes)));
+    const int splits0 = std::min(want, int(dev::div_ceil(nv, 128)));
+    const int v_chunk = int(dev::div_ceil(dev::div_ceil(nv, splits0), 8)) * 8;
     const int splits = int(dev::div_ceil(nv, v_chunk));
     const int64_t plane = int64_t(nc) * nr * ns;
-    auto partial = ctx.empty<cfloat, 1>({int64_t(splits) * (two ? 2 : 1) * plane});
+    auto partial = ctx.empty<cfloat, 1>({int64_t(splits) * plane});
+    auto voxels = ctx.empty<kernels::SpiralVoxel, 1>({nv});
+    {
+        KernelScope ks(ctx, "spiral_voxels");
+        kernels::spiral_voxels<<<dev::div_ceil(nv, 256), 256, 0, ctx.stream()>>>(dev::tissue_view(p), t.delta_t, voxels.data());
+        check_launch("spiral_voxels");
+    }
     {
         KernelScope ks(ctx, "spiral_sum_mfma");
         const dim3 grid(nr, splits, passes);
-        const auto tv = dev::tissue_view(p);
-        hipStream_t s = ctx.stream();
-        const bool full = ns % (16 * tiles) == 0;
-        auto launch = [&](auto two_c, auto lo_c) {
-            constexpr bool TWO = decltype(two_c)::value;
-            constexpr bool LO = decltype(lo_c)::value;
-            if (full) {
-                kernels::spiral_sum_mfma<TWO, LO, tiles, true><<<grid, 64, 0, s>>>(
-                    tv, A, TWO ? Ab : nullptr, coils, nc, t.delta_k.data(), nr, ns, t.delta_t, v_chunk, partial.data());
-            } else {
-                kernels::spiral_sum_mfma<TWO, LO, tiles, false><<<grid, 64, 0, s>>>(
-                    tv, A, TWO ? Ab : nullptr, coils, nc, t.delta_k.data(), nr, ns, t.delta_t, v_chunk, partial.data());
-            }
+        const auto launch = [&](auto ct_c, auto rt_c, auto two_c, auto lo_c) {
+            kernels::spiral_sum_split<decltype(ct_c)::value, decltype(rt_c)::value, decltype(two_c)::value, decltype(lo_c)::value>
+                <<<grid, 64, 0, ctx.stream()>>>(voxels.data(), nv, A, Ab, coils, nc, t.delta_k.data(), nr, ns, tbits,
+                                                v_chunk, partial.data());
         };
-        if (two) {
-            if (lo) launch(std::true_type {}, std::true_type {});
-            else launch(std::true_type {}, std::false_type {});
-        } else {
-            if (lo) launch(std::false_type {}, std::true_type {});
-            else launch(std::false_type {}, std::false_type {});
-        }
+        const auto with_lo = [&](auto ct_c, auto rt_c, auto two_c) {
+            if (lo) launch(ct_c, rt_c, two_c, std::true_type {});
+            else launch(ct_c, rt_c, two_c, std::false_type {});
+        };
+        const auto with_ct = [&](auto rt_c, auto two_c) {
+            if (ct == 2) with_lo(std::integral_constant<int, 2> {}, rt_c, two_c);
+            else with_lo(std::integral_constant<int, 1> {}, rt_c, two_c);
+        };
+        if (two) with_ct(std::integral_constant<int, 2> {}, std::true_type {});
+        else if (rt == 2) with_ct(std::integral_constant<int, 2> {}, std::false_type {});
+        else with_ct(std::integral_constant<int, 1> {}, std::false_type {});
         check_launch("spiral_sum_mfma");
     }
-    {
-        KernelScope ks(ctx, "spiral_sum_reduce");
-        const int64_t blocks = std::min<int64_t>(dev::div_ceil(plane, int64_t(256)), 8192);
-        if (two) kernels::spiral_sum_reduce<true><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
-        else kernels::spiral_sum_reduce<false><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
-        check_launch("spiral_sum_reduce");
-    }
+    KernelScope ks(ctx, "spiral_sum_reduce");
+    const int64_t blocks = std::min<int64_t>(dev::div_ceil(plane, int64_t(256)), 8192);
+    kernels::spiral_sum_reduce<<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, out);
+    check_launch("spiral_sum_reduce");
     return true;
 }
 
