@@ -17,8 +17,6 @@ struct alignas(16) SpiralVoxel {
     float pad[2];
 };
 
-__global__ void spiral_voxels(dev::TissueView t, float dt, SpiralVoxel* __restrict__ out);
-
 // Turns per sample of a voxel; dkx, dky: delta_k / 2 pi
 __device__ __forceinline__ double spiral_turns(const SpiralVoxel& v, double dkx, double dky) {
     return fma(dkx, double(v.x), fma(dky, double(v.y), v.turns));
@@ -36,4 +34,8 @@ __device__ __forceinline__ cfloat spiral_phasor(float log2_mag, double turns) {
 }
 
 }  // namespace kernels
+
+// The voxels' constants, on the context's stream (signal_spiral_mfma.hip)
+Array<kernels::SpiralVoxel, 1> spiral_voxel_table(const CompasContext& ctx, const TissueParameters& p, float dt);
+
 }  // namespace compas

@@ -4,262 +4,276 @@
 //   U[c][v]  = sum_s y[c][r][s] conj(Phi[r][s][v])
 //   U'[c][v] = sum_s (s - ns/2) y[c][r][s] conj(Phi[r][s][v])
 // (jacobian_spiral.hip states Phi and how U, U' combine into the six rows).
-// That is a complex GEMM per readout, rows (coil, U / U') x K = samples x
-// N = voxels, whose B operand conj(Phi) is generated, not stored: Phi is a
-// geometric sequence in s per voxel.  Here it runs on
-// v_mfma_f32_16x16x32_bf16 with BF16 hi + lo operands (FP32 accumulation):
-//   * A (16 real rows per group of four coils: U_re, U_im, U'_re, U'_im rows
-//     of each coil) is built from y once per workgroup and 256-sample chunk,
-//     as (a_re, -a_im) / (a_im, a_re) pairs along the interleaved K split
-//     into hi + lo, and kept in LDS in fragment order (one 16-byte read per
-//     lane, part and K step);
-//   * B (16 voxels per tile) is generated in registers: lane l holds voxel
-//     l % 16 and four consecutive samples 4 (l / 16) + j of each 16-sample
-//     K step, advanced by Phi^16 per step (four complex multiplies) and
-//     restarted from an FP64 phase every 256 samples;
-//   * the 16 x 16 accumulator gives each lane one coil's U and U' of its
-//     voxel, so the per-readout epilogue (the products with conj(m) and
-//     conj(dm_p)) is per lane; coils are summed across the four lane groups
-//     once at the end.
-// Every lane generates only its own B elements: ~10 VALU instructions per
-// (sample, voxel) for the recurrence and the hi/lo split, against ~36 for the
-// FP32 VALU form at four coils.
+// Phi is a geometric sequence in s: with s = sb + S t + n, n < S = 8 KS, Phi_s =
+// Phi_sb E^(S t) E^n and
+//   U  = conj(Phi_sb) sum_t conj(E^(S t)) G_t,   G_t  = sum_n y_(sb + S t + n) conj(E^n)
+//   U' = conj(Phi_sb) sum_t conj(E^(S t)) ((sb + S t - ns/2) G_t + G'_t),
+//                                              G'_t = sum_n n y_(sb + S t + n) conj(E^n).
+// G and G' are a complex GEMM, rows (coil, t) x K = n x N = voxels, whose B
+// operand has S generated elements per voxel and readout instead of ns; the
+// sums over t are Horner's rule on the accumulators.  It runs on
+// v_mfma_f32_32x32x16_bf16 with BF16 hi + lo operands (FP32 accumulation):
+//   * A: four row tiles (real and imaginary parts of G and of G') of 32 (coil,
+//     t) rows, written once per call in fragment order by spiral_y_fragments
+//     and copied to LDS per readout, the next readout's behind the current one;
+//   * B: lane l holds voxel l % 32 and samples n = 8 ks + 4 (l / 32) + j of K
+//     step ks, advanced by E^8 per step, in registers; T tiles of 32 voxels per
+//     wave share the A fragments;
+//   * the rows are ordered so that a lane's sixteen accumulator elements are
+//     two coils with T8's eight t each, or four coils with four: the sums over
+//     t and over the lane's coils (with conj(C)) need no exchange, and the
+//     products with conj(m) and conj(dm_p) are done once per readout.
+// Sample blocks of S T and coil groups repeat the two stages within a readout.
 //
-// Layout of v_mfma_f32_16x16x32_bf16 (wave64): lane l supplies row (A) or
-// column (B) l % 16 and K elements 8 (l / 16) .. 8 (l / 16) + 7; the result
-// element j of lane l is row 4 (l / 16) + j, column l % 16.
+// What bounds it: MFMA (47% of the cycles) and VALU (54%) issue, which overlap
+// little because a barrier per readout keeps the waves of a CU in step, at 1.9
+// GHz.  50176 voxels x 1120 readouts x 512 samples, 4 coils: 14.9 -> 5.6 ms
+// against a form that generated every sample's element; 20000 x 500 x 128 854
+// -> 670 us, x 16 452 -> 351 us.
+//
+// Layout of v_mfma_f32_32x32x16_bf16 (wave64): lane l supplies row (A) or
+// column (B) l % 32 and K elements 8 (l / 32) .. + 7; result element e of lane l
+// is row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32.
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "compas/device/common.h"
 #include "compas/device/mfma_tile.h"
+#include "compas/device/spiral_phasor.h"
 #include "compas/internal.h"
 
 namespace compas {
 namespace kernels {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int SHM_WAVES = 4;  // waves per workgroup
-constexpr int SHM_CHUNK = 256;  // samples of y staged in LDS at a time; Phi restarts at each chunk
+constexpr int SHM_TILES = 4;  // row tiles: G_re, G_im, G'_re, G'_im
 
-__device__ inline mfma::bf16x8 as_bf16x8(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) {
-    const uint4 w = {w0, w1, w2, w3};
-    return __builtin_bit_cast(mfma::bf16x8, w);
+// Coil (of its group) and t of row tile row `row`
+template<bool T8>
+__device__ __forceinline__ void shm_row(int row, int& c, int& t) {
+    const int a = row >> 3, h = (row >> 2) & 1, b = row & 3;
+    c = T8 ? 2 * h + (a >> 1) : 4 * h + a;
+    t = T8 ? 4 * (a & 1) + b : b;
 }
 
-// Phi at sample s: exp((ns/2 - s) dt R2) exp(i (phi0 + s theta)), phase in FP64
-__device__ inline cfloat spiral_phi(double phi0, double theta, float R2, float dt, int ns, int s) {
-    const float mag = expf((0.5f * float(ns) - float(s)) * dt * R2);
-    return dev::polar_reduced(mag, fma(double(s), theta, phi0));
-}
-
-// Partial J^H.y over readouts [r0, r1): partial[chunk * groups + group][p][v].
-// Grid (ceil(nv / (16 T SHM_WAVES)), readout chunks), block 64 SHM_WAVES.  G
-// groups of four coils share the generated operand.
-template<int G, int T, bool LO>
-__global__ void __launch_bounds__(64 * SHM_WAVES) spiral_hermitian_mfma(
-    dev::TissueView t, const cfloat* __restrict__ m, const cfloat* __restrict__ dT1,
-    const cfloat* __restrict__ dT2, const cfloat* __restrict__ dB1, const cfloat* __restrict__ dB0,
-    const cfloat* __restrict__ coils, int nc, const cfloat* __restrict__ y, const cfloat* __restrict__ k_start,
-    const cfloat* __restrict__ delta_k, int nr, int ns, float dt, int r_chunk, cfloat* __restrict__ partial) {
+// A fragments frag[readout][block][K step][tile][hi, lo][lane], block = sample
+// block x coil group; grid (nr, blocks), block 64 KS.
+template<int KS, bool T8, bool LO>
+__global__ void __launch_bounds__(64 * KS) spiral_y_fragments(
+    const cfloat* __restrict__ y, int nc, int nr, int ns, int groups, uint4* __restrict__ frag) {
     constexpr int P = LO ? mfma::P_BF16X3 : mfma::P_BF16X1;
-    constexpr int KSTEPS = SHM_CHUNK / 16;
-    // A fragments of the chunk in fragment order: [group][K step][lane] hi, lo
-    __shared__ uint4 afrag_hi[G][KSTEPS][64];
-    __shared__ uint4 afrag_lo[LO ? G : 1][LO ? KSTEPS : 1][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n = lane & 15, g = lane >> 4;
-    const int nv = t.nvoxels;
-    const int r0 = blockIdx.y * r_chunk, r1 = min(nr, r0 + r_chunk);
-    const int vbase = (blockIdx.x * SHM_WAVES + wave) * (16 * T);
-
-    // voxel constants of the lane's voxel in each tile (out-of-range voxels read voxel 0)
-    int vt[T];
-    bool okt[T];
-    float R2[T], T1v[T], T2v[T];
-    double xv[T], yv[T], B0v[T];
-    cfloat rho[T], Cg[T][G];
+    constexpr int S = 8 * KS, T = T8 ? 8 : 4, COILS = T8 ? 4 : 8, PARTS = LO ? 2 : 1;
+    const int lane = threadIdx.x & 63, ks = threadIdx.x >> 6;
+    const int r = blockIdx.x, block = blockIdx.y;
+    int c, t;
+    shm_row<T8>(lane & 31, c, t);
+    c += COILS * (block % groups);
+    const int n0 = 8 * ks + 4 * (lane >> 5);
+    const int s0 = (block / groups) * (S * T) + S * t + n0;
+    uint32_t hi[SHM_TILES][4], lo[SHM_TILES][4];
 #pragma unroll
-    for (int ti = 0; ti < T; ti++) {
-        const int v = vbase + 16 * ti + n;
-        okt[ti] = v < nv;
-        const int vv = okt[ti] ? v : 0;
-        vt[ti] = vv;
-        T1v[ti] = t.T1(vv);
-        T2v[ti] = t.T2(vv);
-        R2[ti] = 1.0f / T2v[ti];
-        xv[ti] = t.x(vv);
-        yv[ti] = t.y(vv);
-        B0v[ti] = t.B0(vv);
-        rho[ti] = t.rho(vv);
-#pragma unroll
-        for (int gi = 0; gi < G; gi++) {
-            const int c = 4 * gi + g;
-            Cg[ti][gi] = c < nc ? coils[size_t(c) * nv + vv] : cfloat {0, 0};
-        }
+    for (int j = 0; j < 4; j++) {
+        cfloat v = {0.0f, 0.0f};
+        if (c < nc && s0 + j < ns) v = y[(size_t(c) * nr + r) * ns + s0 + j];
+        const cfloat w = v * float(n0 + j);
+        mfma::split_pair<P>(v.re, v.im, hi[0][j], lo[0][j]);
+        mfma::split_pair<P>(v.im, -v.re, hi[1][j], lo[1][j]);
+        mfma::split_pair<P>(w.re, w.im, hi[2][j], lo[2][j]);
+        mfma::split_pair<P>(w.im, -w.re, hi[3][j], lo[3][j]);
     }
-    // per-coil sums over readouts (the lane's coil 4 gi + g of each group)
-    cfloat g1[T][G], g2[T][G], gb1[T][G], gb0[T][G], gu[T][G];
+    uint4* out = frag + ((size_t(r) * gridDim.y + block) * KS + ks) * (SHM_TILES * PARTS * 64) + lane;
 #pragma unroll
-    for (int ti = 0; ti < T; ti++)
-#pragma unroll
-        for (int gi = 0; gi < G; gi++) g1[ti][gi] = g2[ti][gi] = gb1[ti][gi] = gb0[ti][gi] = gu[ti][gi] = {0, 0};
+    for (int i = 0; i < SHM_TILES; i++) {
+        out[(i * PARTS) * 64] = uint4 {hi[i][0], hi[i][1], hi[i][2], hi[i][3]};
+        if constexpr (LO) out[(i * PARTS + 1) * 64] = uint4 {lo[i][0], lo[i][1], lo[i][2], lo[i][3]};
+    }
+}
 
-    const double half = 0.5 * double(ns) * double(dt);
-    const float sp0 = -0.5f * float(ns);
+// Partial J^H.y over readouts [r0, r1): partial[chunk][p][v].  Grid (ceil(nv /
+// (32 T W)), readout chunks), block 64 W; two fragment buffers of KS 4 PARTS KiB.
+template<int T, int W, int KS, bool T8, bool LO>
+__global__ void __launch_bounds__(64 * W, W / 4) spiral_hermitian_mfma(
+    const SpiralVoxel* __restrict__ voxels, dev::TissueView tissue, const cfloat* __restrict__ m,
+    const cfloat* __restrict__ dT1, const cfloat* __restrict__ dT2, const cfloat* __restrict__ dB1,
+    const cfloat* __restrict__ dB0, const cfloat* __restrict__ coils, int nc, const uint4* __restrict__ frag,
+    int blocks, int groups, const cfloat* __restrict__ k_start, const cfloat* __restrict__ delta_k, int nr, int ns,
+    float dt, int r_chunk, cfloat* __restrict__ partial) {
+    constexpr int P = LO ? mfma::P_BF16X3 : mfma::P_BF16X1;
+    constexpr int S = 8 * KS, NT = T8 ? 8 : 4, NC = T8 ? 2 : 4, PARTS = LO ? 2 : 1;
+    constexpr int FRAG = KS * SHM_TILES * PARTS * 64;  // 16-byte words of a block's fragments
+    __shared__ uint4 lds[2 * FRAG];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane & 31, half = lane >> 5;
+    const int nv = tissue.nvoxels;
+    const int r0 = blockIdx.y * r_chunk, r1 = min(nr, r0 + r_chunk);
+    const int vbase = (blockIdx.x * W + wave) * (32 * T);
+
+    int vt[T];
+    SpiralVoxel vx[T];
+#pragma unroll
+    for (int i = 0; i < T; i++) {
+        vt[i] = min(vbase + 32 * i + col, nv - 1);
+        vx[i] = voxels[vt[i]];
+    }
+    cfloat g1[T], g2[T], gb1[T], gb0[T], gu[T];
+#pragma unroll
+    for (int i = 0; i < T; i++) g1[i] = g2[i] = gb1[i] = gb0[i] = gu[i] = {0.0f, 0.0f};
+
+    // a block's fragments, linear in LDS: each wave copies 1 KiB at a time
+    auto fetch = [&](int item, int buf) {
+        const uint4* from = frag + size_t(item) * FRAG;
+#pragma unroll
+        for (int k = 0; k < FRAG / 64; k += W) {
+            if (FRAG / 64 % W == 0 || k + wave < FRAG / 64) {
+                __builtin_amdgcn_global_load_lds(
+                    reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(uintptr_t(from + (k + wave) * 64 + lane)),
+                    (__attribute__((address_space(3))) uint32_t*)(&lds[buf * FRAG + (k + wave) * 64]), 16, 0, 0);
+            }
+        }
+    };
+    int item = r0 * blocks;
+    const int last = r1 * blocks;
+    int buf = 0;
+    if (item < last) fetch(item, 0);
 
     for (int r = r0; r < r1; r++) {
-        const cfloat dk = delta_k[r], k0 = k_start[r];
-        double theta[T], phi0[T];
-        cfloat step1[T], step16[T];
+        const cfloat dk = delta_k[r];
+        const double dkx = double(dk.re) / dev::TWO_PI, dky = double(dk.im) / dev::TWO_PI;
+        const double k0x = double(k_start[r].re) / dev::TWO_PI;
+        cfloat V[T], Vp[T];
 #pragma unroll
-        for (int ti = 0; ti < T; ti++) {
-            theta[ti] = double(dk.re) * xv[ti] + double(dk.im) * yv[ti] + double(dt) * dev::TWO_PI * B0v[ti];
-            phi0[ti] = -half * dev::TWO_PI * B0v[ti] + double(k0.re) * xv[ti];
-            step1[ti] = dev::polar_reduced(expf(-dt * R2[ti]), theta[ti]);
-            step16[ti] = dev::polar_reduced(expf(-16.0f * dt * R2[ti]), 16.0 * theta[ti]);
+        for (int i = 0; i < T; i++) V[i] = Vp[i] = {0.0f, 0.0f};
+        double turns[T];
+        cfloat e1[T], e4[T], e8[T], eS[T];
+#pragma unroll
+        for (int i = 0; i < T; i++) {
+            turns[i] = spiral_turns(vx[i], dkx, dky);
+            e1[i] = spiral_phasor(vx[i].decay, turns[i]);
+            e4[i] = spiral_phasor(float(4 * half) * vx[i].decay, double(4 * half) * turns[i]);
+            e8[i] = spiral_phasor(8.0f * vx[i].decay, 8.0 * turns[i]);
+            eS[i] = spiral_phasor(float(S) * vx[i].decay, double(S) * turns[i]);
         }
-        f32x4 acc[T][G];
-#pragma unroll
-        for (int ti = 0; ti < T; ti++)
-#pragma unroll
-            for (int gi = 0; gi < G; gi++) acc[ti][gi] = f32x4 {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int block = 0; block < blocks; block++, item++) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's part of the block's copy
+            __syncthreads();                                   // everyone's; and the other buffer has been read
+            if (item + 1 < last) fetch(item + 1, buf ^ 1);
+            const uint4* a = &lds[buf * FRAG + lane];
+            buf ^= 1;
 
-        for (int sc = 0; sc < ns; sc += SHM_CHUNK) {
-            __syncthreads();  // the previous chunk's fragments have been read
-            // A fragment of (group gi, K step ks, lane fl): row fl % 16 = coil 4 gi + row / 4 and
-            // (U_re, U_im, U'_re, U'_im)[row % 4], samples sc + 16 ks + 4 (fl / 16) + j, as
-            // (a_re, -a_im) / (a_im, a_re) pairs split into BF16 hi + lo
-            for (int e = threadIdx.x; e < G * KSTEPS * 64; e += 64 * SHM_WAVES) {
-                const int fl = e & 63, ks = (e >> 6) % KSTEPS, gi = e / (64 * KSTEPS);
-                const int row = fl & 15, c = 4 * gi + (row >> 2), q = row & 3;
-                const int s0 = sc + 16 * ks + 4 * (fl >> 4);
-                uint32_t hw[4], lw[4];
+            f32x16 acc[T][SHM_TILES];
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int s = s0 + j;
-                    cfloat a = {0.0f, 0.0f};
-                    if (c < nc && s < ns) a = y[(size_t(c) * nr + r) * ns + s];
-                    if (q >= 2) a = a * (float(s) + sp0);
-                    const float e0 = (q & 1) ? a.im : a.re;
-                    const float e1 = (q & 1) ? a.re : -a.im;
-                    mfma::split_pair<P>(e0, e1, hw[j], lw[j]);
-                }
-                afrag_hi[gi][ks][fl] = uint4 {hw[0], hw[1], hw[2], hw[3]};
-                if constexpr (LO) afrag_lo[gi][ks][fl] = uint4 {lw[0], lw[1], lw[2], lw[3]};
-            }
-            __syncthreads();
-
-            // Phi at the lane's four samples of the first K step of the chunk
+            for (int i = 0; i < T; i++)
+#pragma unroll
+                for (int k = 0; k < SHM_TILES; k++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[i][k][e] = 0.0f;
             cfloat ph[T][4];
 #pragma unroll
-            for (int ti = 0; ti < T; ti++) {
-                ph[ti][0] = spiral_phi(phi0[ti], theta[ti], R2[ti], dt, ns, sc + 4 * g);
+            for (int i = 0; i < T; i++) {
+                ph[i][0] = e4[i];
 #pragma unroll
-                for (int j = 1; j < 4; j++) ph[ti][j] = dev::cmul(ph[ti][j - 1], step1[ti]);
+                for (int j = 1; j < 4; j++) ph[i][j] = dev::cmul(ph[i][j - 1], e1[i]);
             }
-            const int kend = min(SHM_CHUNK, ns - sc);
-            for (int ks = 0; ks < kend; ks += 16) {
-                mfma::bf16x8 ahi[G], alo[G];
+#pragma unroll 2
+            for (int ks = 0; ks < KS; ks++) {
+                mfma::bf16x8 bh[T], bl[T];
 #pragma unroll
-                for (int gi = 0; gi < G; gi++) {
-                    ahi[gi] = __builtin_bit_cast(mfma::bf16x8, afrag_hi[gi][ks >> 4][lane]);
-                    if constexpr (LO) alo[gi] = __builtin_bit_cast(mfma::bf16x8, afrag_lo[gi][ks >> 4][lane]);
-                }
-#pragma unroll
-                for (int ti = 0; ti < T; ti++) {
-                    // B: conj(Phi) of voxel n at the lane's four samples, as (re, im) pairs
+                for (int i = 0; i < T; i++) {
                     uint32_t hw[4], lw[4];
 #pragma unroll
-                    for (int j = 0; j < 4; j++) mfma::split_pair<P>(ph[ti][j].re, -ph[ti][j].im, hw[j], lw[j]);
-                    const mfma::bf16x8 bhi = as_bf16x8(hw[0], hw[1], hw[2], hw[3]);
-                    const mfma::bf16x8 blo = as_bf16x8(lw[0], lw[1], lw[2], lw[3]);
-#pragma unroll
-                    for (int gi = 0; gi < G; gi++) {
-                        acc[ti][gi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[gi], bhi, acc[ti][gi], 0, 0, 0);
-                        if constexpr (LO) {
-                            acc[ti][gi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[gi], blo, acc[ti][gi], 0, 0, 0);
-                            acc[ti][gi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo[gi], bhi, acc[ti][gi], 0, 0, 0);
-                        }
+                    for (int j = 0; j < 4; j++) {
+                        mfma::split_pair<P>(ph[i][j].re, ph[i][j].im, hw[j], lw[j]);
+                        ph[i][j] = dev::cmul(ph[i][j], e8[i]);
                     }
+                    bh[i] = __builtin_bit_cast(mfma::bf16x8, uint4 {hw[0], hw[1], hw[2], hw[3]});
+                    bl[i] = __builtin_bit_cast(mfma::bf16x8, uint4 {lw[0], lw[1], lw[2], lw[3]});
+                }
 #pragma unroll
-                    for (int j = 0; j < 4; j++) ph[ti][j] = dev::cmul(ph[ti][j], step16[ti]);
+                for (int k = 0; k < SHM_TILES; k++) {
+                    const mfma::bf16x8 ah = __builtin_bit_cast(mfma::bf16x8, a[((ks * SHM_TILES + k) * PARTS) * 64]);
+#pragma unroll
+                    for (int i = 0; i < T; i++) {
+                        acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh[i], acc[i][k], 0, 0, 0);
+                        if constexpr (LO) acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl[i], acc[i][k], 0, 0, 0);
+                    }
+                    if constexpr (LO) {
+                        const mfma::bf16x8 al = __builtin_bit_cast(mfma::bf16x8, a[((ks * SHM_TILES + k) * PARTS + 1) * 64]);
+#pragma unroll
+                        for (int i = 0; i < T; i++)
+                            acc[i][k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh[i], acc[i][k], 0, 0, 0);
+                    }
                 }
             }
-        }
 
-        // readout epilogue: the lane holds U, U' of coil 4 gi + g for its voxel
+            // sums over t (Horner in conj(E^S)), conj(Phi_sb), the lane's coils
+            const int sb = (block / groups) * (S * NT), c0 = (block % groups) * (2 * NC) + NC * half;
 #pragma unroll
-        for (int ti = 0; ti < T; ti++) {
-            const size_t i = size_t(r) * nv + vt[ti];
-            const cfloat me = m[i], a1 = dT1[i], a2 = dT2[i], ab1 = dB1[i], ab0 = dB0[i];
-            const float kT2 = dt * R2[ti] * R2[ti];
-            const float kB0 = -dev::TWO_PI_F * dt;
+            for (int i = 0; i < T; i++) {
+                const double first = fma(k0x, double(vx[i].x), fma(double(sb), turns[i], -0.5 * double(ns) * vx[i].turns));
+                const cfloat phi = spiral_phasor((float(sb) - 0.5f * float(ns)) * vx[i].decay, first);
+                cfloat sum = {0.0f, 0.0f}, sump = {0.0f, 0.0f};
 #pragma unroll
-            for (int gi = 0; gi < G; gi++) {
-                const cfloat U = {acc[ti][gi][0], acc[ti][gi][1]};
-                const cfloat Up = {acc[ti][gi][2], acc[ti][gi][3]};
-                g1[ti][gi] = dev::cfma_conj(U, a1, g1[ti][gi]);
-                g2[ti][gi] = dev::cfma_conj(U, a2, g2[ti][gi]);
-                g2[ti][gi] = dev::cfma_conj(Up * kT2, me, g2[ti][gi]);
-                gb1[ti][gi] = dev::cfma_conj(U, ab1, gb1[ti][gi]);
-                gb0[ti][gi] = dev::cfma_conj(U, ab0, gb0[ti][gi]);
-                gb0[ti][gi] = dev::cfma_conj(cfloat {-Up.im * kB0, Up.re * kB0}, me, gb0[ti][gi]);
-                gu[ti][gi] = dev::cfma_conj(U, me, gu[ti][gi]);
+                for (int k = 0; k < NC; k++) {
+                    cfloat U, Up;
+#pragma unroll
+                    for (int t = NT - 1; t >= 0; t--) {
+                        const int e = NT * k + t;
+                        const float tau = float(sb + S * t) - 0.5f * float(ns);
+                        const cfloat G = {acc[i][0][e], acc[i][1][e]};
+                        const cfloat H = {fmaf(tau, G.re, acc[i][2][e]), fmaf(tau, G.im, acc[i][3][e])};
+                        U = t == NT - 1 ? G : dev::cfma_conj(U, eS[i], G);
+                        Up = t == NT - 1 ? H : dev::cfma_conj(Up, eS[i], H);
+                    }
+                    cfloat C = coils[size_t(min(c0 + k, nc - 1)) * nv + vt[i]];
+                    if (c0 + k >= nc) C = {0.0f, 0.0f};
+                    sum = dev::cfma_conj(U, C, sum);
+                    sump = dev::cfma_conj(Up, C, sump);
+                }
+                V[i] = dev::cfma_conj(sum, phi, V[i]);
+                Vp[i] = dev::cfma_conj(sump, phi, Vp[i]);
             }
+        }
+#pragma unroll
+        for (int i = 0; i < T; i++) {
+            const size_t at = size_t(r) * nv + vt[i];
+            const cfloat me = m[at], a1 = dT1[at], a2 = dT2[at], ab1 = dB1[at], ab0 = dB0[at];
+            const float R2 = 1.0f / vx[i].T2;
+            const float kT2 = dt * R2 * R2, kB0 = -dev::TWO_PI_F * dt;
+            g1[i] = dev::cfma_conj(V[i], a1, g1[i]);
+            g2[i] = dev::cfma_conj(V[i], a2, g2[i]);
+            g2[i] = dev::cfma_conj(Vp[i] * kT2, me, g2[i]);
+            gb1[i] = dev::cfma_conj(V[i], ab1, gb1[i]);
+            gb0[i] = dev::cfma_conj(V[i], ab0, gb0[i]);
+            gb0[i] = dev::cfma_conj(cfloat {-Vp[i].im * kB0, Vp[i].re * kB0}, me, gb0[i]);
+            gu[i] = dev::cfma_conj(V[i], me, gu[i]);
         }
     }
 
-    // fold the lane's coils, sum the four lane groups (coils 4 gi + g), store
+    // the two halves hold different coils of one voxel
 #pragma unroll
-    for (int ti = 0; ti < T; ti++) {
-        cfloat out[5];
-#pragma unroll
-        for (int p = 0; p < 5; p++) out[p] = {0, 0};
-#pragma unroll
-        for (int gi = 0; gi < G; gi++) {
-            const cfloat C = Cg[ti][gi];
-            const cfloat rc = dev::cmul(rho[ti], C);
-            out[0] = out[0] + dev::cmul(conj(rc * T1v[ti]), g1[ti][gi]);
-            out[1] = out[1] + dev::cmul(conj(rc * T2v[ti]), g2[ti][gi]);
-            out[2] = out[2] + dev::cmul(conj(rc), gb1[ti][gi]);
-            out[3] = out[3] + dev::cmul(conj(rc), gb0[ti][gi]);
-            out[4] = out[4] + dev::cmul(conj(C), gu[ti][gi]);
-        }
+    for (int i = 0; i < T; i++) {
+        const cfloat rho = tissue.rho(vt[i]);
+        cfloat o[5] = {dev::cmul(conj(rho * tissue.T1(vt[i])), g1[i]), dev::cmul(conj(rho * vx[i].T2), g2[i]),
+                       dev::cmul(conj(rho), gb1[i]), dev::cmul(conj(rho), gb0[i]), gu[i]};
 #pragma unroll
         for (int p = 0; p < 5; p++) {
-            out[p].re += __shfl_xor(out[p].re, 16);
-            out[p].im += __shfl_xor(out[p].im, 16);
-            out[p].re += __shfl_xor(out[p].re, 32);
-            out[p].im += __shfl_xor(out[p].im, 32);
+            o[p].re += __shfl_xor(o[p].re, 32);
+            o[p].im += __shfl_xor(o[p].im, 32);
         }
-        if (g == 0 && okt[ti]) {
-            const int v = vbase + 16 * ti + n;
+        const int v = vbase + 32 * i + col;
+        if (half == 0 && v < nv) {
             cfloat* dst = partial + size_t(blockIdx.y) * 6 * size_t(nv) + v;
 #pragma unroll
-            for (int p = 0; p < 5; p++) dst[size_t(p) * nv] = out[p];
-            dst[size_t(5) * nv] = dev::cmul(out[4], cfloat {0.0f, -1.0f});
+            for (int p = 0; p < 5; p++) dst[size_t(p) * nv] = o[p];
+            dst[size_t(5) * nv] = dev::cmul(o[4], cfloat {0.0f, -1.0f});
         }
     }
 }
 
 }  // namespace kernels
-
-namespace {
-
-constexpr int SHM_T = 2;  // 16-voxel tiles per wave
-
-template<int G, bool LO>
-void launch_shm(dim3 grid, hipStream_t s, const dev::TissueView& tv, const cfloat* m, const cfloat* d1, const cfloat* d2,
-                const cfloat* db1, const cfloat* db0, const cfloat* coils, int nc, const cfloat* y, const cfloat* k0,
-                const cfloat* dk, int nr, int ns, float dt, int r_chunk, cfloat* partial) {
-    kernels::spiral_hermitian_mfma<G, SHM_T, LO><<<grid, 64 * kernels::SHM_WAVES, 0, s>>>(
-        tv, m, d1, d2, db1, db0, coils, nc, y, k0, dk, nr, ns, dt, r_chunk, partial);
-}
-
-}  // namespace
 
 bool spiral_hermitian_mfma(
     const CompasContext& ctx, const TissueParameters& p, const cfloat* m, const cfloat* d1, const cfloat* d2,
@@ -269,29 +283,68 @@ bool spiral_hermitian_mfma(
     if (nc > 8) return false;  // more coils: the VALU form
     const bool lo = precision == ContractionPrecision::BF16x3 || precision == ContractionPrecision::FP16x3;
     const int nr = traj.nreadouts, ns = traj.samples_per_readout, nv = p.nvoxels;
-    const int vblocks = int(dev::div_ceil(nv, 16 * SHM_T * kernels::SHM_WAVES));
-    // readout chunks so that about eight waves per SIMD are in the grid
-    const int want = std::max(1, std::min(nr, int(dev::div_ceil(8 * 1024, int64_t(vblocks) * kernels::SHM_WAVES))));
-    const int r_chunk = int(dev::div_ceil(nr, want));
-    const int chunks = int(dev::div_ceil(nr, r_chunk));
-    auto partial = ctx.empty<cfloat, 1>({int64_t(chunks) * 6 * nv});
-    const auto tv = dev::tissue_view(p);
-    {
-        KernelScope ks(ctx, "spiral_hermitian_mfma");
-        const dim3 grid(vblocks, chunks);
-        hipStream_t s = ctx.stream();
-        const cfloat *k0 = traj.k_start.data(), *dk = traj.delta_k.data();
-        const float dt = traj.delta_t;
-        if (nc <= 4) {
-            if (lo) launch_shm<1, true>(grid, s, tv, m, d1, d2, db1, db0, coils, nc, y, k0, dk, nr, ns, dt, r_chunk, partial.data());
-            else launch_shm<1, false>(grid, s, tv, m, d1, d2, db1, db0, coils, nc, y, k0, dk, nr, ns, dt, r_chunk, partial.data());
-        } else {
-            if (lo) launch_shm<2, true>(grid, s, tv, m, d1, d2, db1, db0, coils, nc, y, k0, dk, nr, ns, dt, r_chunk, partial.data());
-            else launch_shm<2, false>(grid, s, tv, m, d1, d2, db1, db0, coils, nc, y, k0, dk, nr, ns, dt, r_chunk, partial.data());
+    // one voxel tile in each of twelve waves, three to a SIMD (at 4 coils x 1120 x
+    // 512 over 50176 voxels 5.7 ms; two tiles in each of eight waves spilled, 5.9;
+    // sixteen waves 6.3)
+    constexpr int T = 1, W = 12;
+    // four t of the smallest S that holds the samples, eight t of S = 64 for more
+    // than 256, blocks of 512 beyond
+    const int ks = ns <= 32 ? 1 : ns <= 64 ? 2 : ns <= 128 ? 4 : 8;
+    const bool t8 = ns > 256;
+    const int groups = int(dev::div_ceil(nc, t8 ? 4 : 8));
+    const int blocks = groups * int(dev::div_ceil(ns, 8 * ks * (t8 ? 8 : 4)));
+    const size_t words = size_t(ks) * kernels::SHM_TILES * (lo ? 2 : 1) * 64;
+    auto frag = ctx.empty<uint4, 1>({int64_t(nr) * blocks * int64_t(words)});
+    auto voxels = spiral_voxel_table(ctx, p, traj.delta_t);
+    const int vblocks = int(dev::div_ceil(nv, 32 * T * W));
+    const auto run = [&](auto ks_c, auto t8_c, auto lo_c) {
+        constexpr int KS = decltype(ks_c)::value;
+        constexpr bool T8 = decltype(t8_c)::value, LO = decltype(lo_c)::value;
+        {
+            KernelScope scope(ctx, "spiral_y_fragments");
+            kernels::spiral_y_fragments<KS, T8, LO><<<dim3(nr, blocks), 64 * KS, 0, ctx.stream()>>>(
+                y, nc, nr, ns, groups, frag.data());
+            check_launch("spiral_y_fragments");
         }
-        check_launch("spiral_hermitian_mfma");
-    }
-    spiral_hermitian_reduce_partials(ctx, partial.data(), chunks, nv, JHy);
+        // readout chunks: the fewest rounds of resident workgroups times a chunk's
+        // readouts (and two readouts' worth of beginning and end)
+        static const int resident = [] {
+            int n = 0;
+            COMPAS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &n, kernels::spiral_hermitian_mfma<T, W, KS, T8, LO>, 64 * W, 0));
+            return std::max(1, n);
+        }();
+        const int64_t slots = int64_t(simd_count(ctx.device()) / 4) * resident;
+        int r_chunk = nr;
+        int64_t best = INT64_MAX;
+        for (int n = 1; n <= nr && (n == 1 || int64_t(n) * vblocks <= 8 * slots); n++) {
+            const int size = int(dev::div_ceil(nr, n));
+            const int64_t cost = int64_t(dev::div_ceil(int64_t(dev::div_ceil(nr, size)) * vblocks, slots)) * (size + 2);
+            if (cost < best) {
+                best = cost;
+                r_chunk = size;
+            }
+        }
+        const int chunks = int(dev::div_ceil(nr, r_chunk));
+        auto partial = ctx.empty<cfloat, 1>({int64_t(chunks) * 6 * nv});
+        {
+            KernelScope scope(ctx, "spiral_hermitian_mfma");
+            kernels::spiral_hermitian_mfma<T, W, KS, T8, LO><<<dim3(vblocks, chunks), 64 * W, 0, ctx.stream()>>>(
+                voxels.data(), dev::tissue_view(p), m, d1, d2, db1, db0, coils, nc, frag.data(), blocks, groups,
+                traj.k_start.data(), traj.delta_k.data(), nr, ns, traj.delta_t, r_chunk, partial.data());
+            check_launch("spiral_hermitian_mfma");
+        }
+        spiral_hermitian_reduce_partials(ctx, partial.data(), chunks, nv, JHy);
+    };
+    const auto with_lo = [&](auto ks_c, auto t8_c) {
+        if (lo) run(ks_c, t8_c, std::true_type {});
+        else run(ks_c, t8_c, std::false_type {});
+    };
+    if (ks == 1) with_lo(std::integral_constant<int, 1> {}, std::false_type {});
+    else if (ks == 2) with_lo(std::integral_constant<int, 2> {}, std::false_type {});
+    else if (ks == 4) with_lo(std::integral_constant<int, 4> {}, std::false_type {});
+    else if (!t8) with_lo(std::integral_constant<int, 8> {}, std::false_type {});
+    else with_lo(std::integral_constant<int, 8> {}, std::true_type {});
     return true;
 }
 

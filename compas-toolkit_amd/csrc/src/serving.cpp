@@ -309,13 +309,16 @@ size_t Server::estimate_bytes(const ServeRequest& r) const {
         }
     }
     if (r.kind == RequestKind::SimulateSignal) {
-        bytes += 8 * nc * nr * ns * 17;  // signal + split-K partials
+        // signal + partial sums: split-K of the contraction, voxel ranges of the spiral sum
+        const size_t planes = r.cartesian ? 17 : 1 + std::min<size_t>(8192 / std::max<size_t>(nr, 1) + 1, nv / 128 + 1);
+        bytes += 8 * nc * nr * ns * planes;
         bytes += r.cartesian ? 8 * nc * ns * nv : echo;  // operand W, or the spiral amplitudes
     } else {
         const size_t nder = fd_count(r);
         // derivatives (each computed in place over its perturbed simulation),
         // the decay operand and the partial sums of the contraction
         bytes += nder * echo + 16 * nv * ns + 2 * echo;
+        if (!r.cartesian) bytes += nr * (size_t(128) << 10);  // the residual as operand fragments
     }
     return bytes;
 }

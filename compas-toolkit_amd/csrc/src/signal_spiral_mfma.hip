@@ -235,6 +235,14 @@ __global__ void spiral_sum_reduce(const cfloat* __restrict__ partial, int splits
 
 }  // namespace kernels
 
+Array<kernels::SpiralVoxel, 1> spiral_voxel_table(const CompasContext& ctx, const TissueParameters& p, float dt) {
+    auto voxels = ctx.empty<kernels::SpiralVoxel, 1>({p.nvoxels});
+    KernelScope ks(ctx, "spiral_voxels");
+    kernels::spiral_voxels<<<dev::div_ceil(p.nvoxels, 256), 256, 0, ctx.stream()>>>(dev::tissue_view(p), dt, voxels.data());
+    check_launch("spiral_voxels");
+    return voxels;
+}
+
 bool spiral_sum_mfma(
     const CompasContext& ctx, const TissueParameters& p, const cfloat* A, const cfloat* Ab, const cfloat* coils,
     int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out) {
@@ -260,12 +268,7 @@ bool spiral_sum_mfma(
     const int splits = int(dev::div_ceil(nv, v_chunk));
     const int64_t plane = int64_t(nc) * nr * ns;
     auto partial = ctx.empty<cfloat, 1>({int64_t(splits) * plane});
-    auto voxels = ctx.empty<kernels::SpiralVoxel, 1>({nv});
-    {
-        KernelScope ks(ctx, "spiral_voxels");
-        kernels::spiral_voxels<<<dev::div_ceil(nv, 256), 256, 0, ctx.stream()>>>(dev::tissue_view(p), t.delta_t, voxels.data());
-        check_launch("spiral_voxels");
-    }
+    auto voxels = spiral_voxel_table(ctx, p, t.delta_t);
     {
         KernelScope ks(ctx, "spiral_sum_mfma");
         const dim3 grid(nr, splits, passes);
