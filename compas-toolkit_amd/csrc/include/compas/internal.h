@@ -146,9 +146,11 @@ void spiral_hermitian_reduce_partials(const CompasContext& ctx, const cfloat* pa
 int64_t pssfp_scratch_bytes(const CompasContext& ctx, int nz, int nv, int nTR);
 
 // echos[i] += sum over count partial planes of n elements (plane j at
-// partial + j * stride), in FP64, in order
+// partial + j * stride), in FP64, in order; with the table of a train, only if
+// the maps served it (`mapped`) or only if they did not
 void pssfp_sum_groups(
-    const CompasContext& ctx, cfloat* echos, const cfloat* partial, int count, int64_t n, int64_t stride);
+    const CompasContext& ctx, cfloat* echos, const cfloat* partial, int count, int64_t n, int64_t stride,
+    const double* train = nullptr, bool mapped = false);
 
 // Work-table launches of the request server: workgroup b runs items[b].
 //   FISP: item (job, voxel block of 64), every job with max_state == spl,
@@ -180,6 +182,14 @@ void launch_pssfp_map(
     const int2* items, int64_t n);
 void launch_pssfp_unmapped(const CompasContext& ctx, const kernels::PssfpMapArgs& p);
 void pssfp_map_finish(const CompasContext& ctx, const kernels::PssfpMapArgs& p);
+
+// The train's table alone; and the tangents by maps (pssfp_map_tangent.hip):
+// whether they pay for a field set (TangentSet mask), and the pass, which does
+// nothing for trains beyond the maps.
+void pssfp_map_table(const CompasContext& ctx, const kernels::PssfpArgs& a, double* train);
+bool pssfp_map_tangents_pay(int mask, int nTR, int nRF);
+void launch_pssfp_map_tangents(
+    const CompasContext& ctx, int mask, const kernels::PssfpArgs& a, const double* train, cfloat* const* planes);
 
 // Finite-difference pieces of simulate_magnetization_derivative
 // (derivative.cu:11-94): the parameters with `field` moved by `delta` (the

@@ -227,8 +227,12 @@ __global__ void __launch_bounds__(64) pssfp_iso_table(const PssfpTableJob* __res
 }
 
 // echos[i] += sum_j partial[j][i], accumulated in FP64 in slot order
+// (train: nullptr, or the table of a train: nothing is done unless the maps
+// served it, or did not, as `mapped` says)
 __global__ void pssfp_sum_groups_kernel(
-    cfloat* __restrict__ echos, const cfloat* __restrict__ partial, int count, int64_t n, int64_t stride) {
+    cfloat* __restrict__ echos, const cfloat* __restrict__ partial, int count, int64_t n, int64_t stride,
+    const double* train, bool mapped) {
+    if (train != nullptr && (train[1] != 0.0) != mapped) return;
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
         const cfloat e = echos[i];
         double re = e.re, im = e.im;
@@ -244,11 +248,12 @@ __global__ void pssfp_sum_groups_kernel(
 }  // namespace kernels
 
 void pssfp_sum_groups(
-    const CompasContext& ctx, cfloat* echos, const cfloat* partial, int count, int64_t n, int64_t stride) {
+    const CompasContext& ctx, cfloat* echos, const cfloat* partial, int count, int64_t n, int64_t stride,
+    const double* train, bool mapped) {
     if (count <= 0 || n == 0) return;
     KernelScope ks(ctx, "pssfp_sum_groups");
     const int64_t blocks = std::min<int64_t>(dev::div_ceil(n, int64_t(256)), 8192);
-    kernels::pssfp_sum_groups_kernel<<<unsigned(blocks), 256, 0, ctx.stream()>>>(echos, partial, count, n, stride);
+    kernels::pssfp_sum_groups_kernel<<<unsigned(blocks), 256, 0, ctx.stream()>>>(echos, partial, count, n, stride, train, mapped);
     check_launch("pssfp_sum_groups");
 }
 

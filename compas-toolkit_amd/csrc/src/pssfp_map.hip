@@ -370,6 +370,12 @@ int64_t pssfp_map_train_size(int nTR) {
     return int64_t(nTR + 2) * kernels::MAP_ROW;  // the header, the rows, and one read ahead
 }
 
+void pssfp_map_table(const CompasContext& ctx, const kernels::PssfpArgs& a, double* train) {
+    KernelScope ks(ctx, "pssfp_map_train");
+    kernels::pssfp_map_train<<<1, 1024, 0, ctx.stream()>>>(a, train);
+    check_launch("pssfp_map_train");
+}
+
 void pssfp_map_setup(const CompasContext& ctx, kernels::PssfpMapArgs& p, const kernels::PssfpArgs& a, double* train, int zpl) {
     p.a = a;
     p.train = train;
@@ -378,9 +384,7 @@ void pssfp_map_setup(const CompasContext& ctx, kernels::PssfpMapArgs& p, const k
     p.vblocks = int(dev::div_ceil(a.tissue.nvoxels, p.nv_block));
     p.direct_zpl = zpl;
     p.direct_groups = (a.nz + zpl - 1) / zpl;
-    KernelScope ks(ctx, "pssfp_map_train");
-    kernels::pssfp_map_train<<<1, 1024, 0, ctx.stream()>>>(a, train);
-    check_launch("pssfp_map_train");
+    pssfp_map_table(ctx, a, train);
 }
 
 int pssfp_map_partial_planes(const kernels::PssfpMapArgs& p) {

@@ -25,6 +25,9 @@
 // axis term).  The pass can also write the echoes it carries, so a caller
 // that needs the signal and all its derivatives runs the recursion once.
 //
+// This is the form for short trains and waveforms and for flip angles beyond the
+// per-TR maps (pssfp_map_tangent.hip), which carry the others.
+//
 // Layout: as the primal kernel (one wave per block of 64 voxels and group of
 // ZPL <= 4 slice positions, partial sums over z added by a second pass).
 
@@ -306,8 +309,11 @@ __device__ inline void rotate_z_all(Vec3d& m, Vec3d* dm, double c, double s, dou
 
 // grid (ceil(nv / 64), groups in this launch), block 64: one wave per voxel
 // block and group of ZPL slice positions, as the primal kernel.
+// train: nullptr, or the table of a train (pssfp_map.h); the launch does nothing
+// where the maps served it.
 template<int ZPL, int MASK>
-__global__ void __launch_bounds__(64) pssfp_iso_tangents(PssfpArgs a, int group0, TangentPlanes out) {
+__global__ void __launch_bounds__(64) pssfp_iso_tangents(PssfpArgs a, int group0, TangentPlanes out, const double* train) {
+    if (train != nullptr && train[1] != 0.0) return;
     using S = TangentSet<MASK>;
     constexpr int NT = S::nt, NP = S::planes, OFS = int(S::echo);
     static_assert(NT >= 1, "a tangent pass carries at least one tangent");
@@ -496,11 +502,12 @@ using kernels::TM_ECHO;
 using kernels::TM_T1;
 using kernels::TM_T2;
 
-using TangentLauncher = void (*)(kernels::PssfpArgs, int, kernels::TangentPlanes, dim3, hipStream_t);
+using TangentLauncher = void (*)(kernels::PssfpArgs, int, kernels::TangentPlanes, const double*, dim3, hipStream_t);
 
 template<int ZPL, int MASK>
-void launch_tangents(kernels::PssfpArgs a, int group0, kernels::TangentPlanes out, dim3 grid, hipStream_t s) {
-    kernels::pssfp_iso_tangents<ZPL, MASK><<<grid, 64, 0, s>>>(a, group0, out);
+void launch_tangents(
+    kernels::PssfpArgs a, int group0, kernels::TangentPlanes out, const double* train, dim3 grid, hipStream_t s) {
+    kernels::pssfp_iso_tangents<ZPL, MASK><<<grid, 64, 0, s>>>(a, group0, out, train);
 }
 
 template<int ZPL, int MASK>
@@ -584,6 +591,14 @@ void run_pass(const CompasContext& ctx, int mask, const kernels::PssfpArgs& a, c
     TangentLauncher fn;
     if (!layout_for_mask(mask, ctx, nz, nv, nTR, &L, &fn)) COMPAS_ERROR("no tangent kernel for this field set");
     const int64_t plane = int64_t(nTR) * nv;
+    // by maps where they pay and the sub-step form they fall back to would run as
+    // one launch
+    Array<double, 1> table;
+    if (pssfp_map_tangents_pay(mask, nTR, a.nRF) && L.groups <= L.per_launch) {
+        table = ctx.empty<double, 1>({pssfp_map_train_size(nTR)});
+        pssfp_map_table(ctx, a, table.data());
+    }
+    const double* train = table.data();
     const int slots = L.groups > L.per_launch ? L.per_launch : L.groups - 1;
     Array<cfloat, 2> part;  // slot s, plane k at (s * np + k) * plane
     if (slots > 0) part = ctx.empty<cfloat, 2>({int64_t(slots) * np, plane});
@@ -595,13 +610,14 @@ void run_pass(const CompasContext& ctx, int mask, const kernels::PssfpArgs& a, c
         out.rest = g0 == 0 ? part.data() : part.data() + np * plane;
         {
             KernelScope ks(ctx, "pssfp_iso_tangents");
-            fn(a, g0, out, dim3(vblocks, unsigned(count)), ctx.stream());
+            fn(a, g0, out, train, dim3(vblocks, unsigned(count)), ctx.stream());
             check_launch("pssfp_iso_tangents");
         }
         const int summed = g0 == 0 ? count - 1 : count;
         for (int k = 0; k < np; k++)
-            pssfp_sum_groups(ctx, planes[k], part.data() + k * plane, summed, plane, np * plane);
+            pssfp_sum_groups(ctx, planes[k], part.data() + k * plane, summed, plane, np * plane, train, false);
     }
+    if (train != nullptr) launch_pssfp_map_tangents(ctx, mask, a, train, planes);
 }
 
 }  // namespace

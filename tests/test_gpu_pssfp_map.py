@@ -15,6 +15,7 @@ import pytest
 import compas_amd as ca
 from compas_amd import workloads as W
 from gpu_helpers import banner, context, rel
+from test_gpu_parity import central_difference
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +57,32 @@ def test_pssfp_map(oracle, nv, nTR, nz, nRF, deg, phase):
         assert np.array_equal(got, np.zeros_like(got))
     else:
         assert rel(got, want) < TOL
+
+
+FIELDS = [(ca.T1, ca.T2, ca.B1, ca.B0), (ca.T1, ca.T2), (ca.T1,), (ca.T2,), (ca.B1,), (ca.B0,)]
+
+
+@pytest.mark.parametrize("fields", FIELDS, ids=lambda f: "".join("T1 T2 B1 B0".split()[i] for i in f))
+@pytest.mark.parametrize("nv,nTR,nz,nRF,deg,phase", [
+    (1, 65, 1, 14, 60.0, 0.0),      # one isochromat
+    (67, 64, 1, 25, 70.0, 0.0),     # 64 voxels to a workgroup, or half of 128
+    (8, 71, 35, 25, 70.0, 0.0),     # several groups; a last chunk that is not full
+    (8, 71, 35, 25, 70.0, 1.1),     # the same with RF phases
+    (3, 66, 130, 12, 45.0, 0.6),    # more positions than a workgroup holds
+    (20, 64, 7, 25, 170.0, 0.4),    # too strong for the maps
+    (5, 20, 7, 8, 60.0, 0.0),       # too short for them
+])
+def test_pssfp_map_tangents(oracle, fields, nv, nTR, nz, nRF, deg, phase):
+    """FP64 maps leave FP32 roundings of the outputs and of up to five partial
+    planes, 3e-7, about 1e-10 per TR of interpolation, and the reference's
+    central differences 1e-8: 1e-6."""
+    banner(f"pssfp map tangents {fields} {nv} voxels {nTR} TRs {nz} positions {nRF} sub-steps {deg} deg phase {phase}")
+    context()
+    n = int(np.ceil(np.sqrt(nv)))
+    t = W.make_tissue(W.SplitMix64(77), n, 20.0, 40.0).slice(0, nv)
+    seq = train(nTR, deg, nz, nRF, phase)
+    p, s = ca.TissueParameters.from_tissue(t), ca.pSSFPSequence.from_sequence(seq)
+    out = [a.collect() for a in ca.simulate_magnetization_tangents(fields, p, s, echos=True)]
+    assert rel(out[0], oracle.pssfp(t, seq, "f64")) < TOL
+    for f, d in zip(fields, out[1:]):
+        assert rel(d, central_difference(oracle.pssfp, t, seq, ["T1", "T2", "B1", "B0"][f])) < 1e-6
