@@ -21,6 +21,7 @@
 //     pass is needed.
 
 #include <cfloat>
+#include <algorithm>
 #include <cmath>
 
 #include <cstdlib>
@@ -29,8 +30,7 @@
 
 #include "compas/device/common.h"
 #include "compas/device/fisp_common.h"
-#include "compas/device/fisp_epg.h"
-#include "compas/device/fisp_real.h"
+#include "compas/device/fisp_launch.h"
 #include "compas/internal.h"
 
 namespace compas {
@@ -73,106 +73,7 @@ __global__ void __launch_bounds__(1024) fisp_rf_table(
     }
 }
 
-template<int SPL, int LPV>
-__global__ void __launch_bounds__(64) fisp_epg(FispArgs a) {
-    const int sub = (LPV > 1) ? int(threadIdx.x % LPV) : 0;
-    const int voxel = (blockIdx.x * 64 + threadIdx.x) / LPV;
-    if (fisp_real_train(a)) return;  // fisp_real runs instead
-    if (voxel >= a.tissue.nvoxels) return;  // whole LPV groups leave together
-    fisp_epg_voxel<SPL, LPV>(a, voxel, sub);
-}
-
 }  // namespace kernels
-
-using FispLauncher = void (*)(kernels::FispArgs, unsigned, hipStream_t);
-
-template<int SPL, int LPV>
-static void launch_fisp(kernels::FispArgs a, unsigned blocks, hipStream_t stream) {
-    kernels::fisp_epg<SPL, LPV><<<blocks, 64, 0, stream>>>(a);
-}
-
-#define COMPAS_FISP_CASE(S, L) \
-    case S:                    \
-        return &launch_fisp<S, L>;
-
-static FispLauncher fisp_launcher_lpv1(int spl) {
-    switch (spl) {
-        COMPAS_FISP_CASE(1, 1)
-        COMPAS_FISP_CASE(2, 1)
-        COMPAS_FISP_CASE(3, 1)
-        COMPAS_FISP_CASE(4, 1)
-        COMPAS_FISP_CASE(5, 1)
-        COMPAS_FISP_CASE(6, 1)
-        COMPAS_FISP_CASE(7, 1)
-        COMPAS_FISP_CASE(8, 1)
-        COMPAS_FISP_CASE(9, 1)
-        COMPAS_FISP_CASE(10, 1)
-        COMPAS_FISP_CASE(11, 1)
-        COMPAS_FISP_CASE(12, 1)
-        COMPAS_FISP_CASE(13, 1)
-        COMPAS_FISP_CASE(14, 1)
-        COMPAS_FISP_CASE(15, 1)
-        COMPAS_FISP_CASE(16, 1)
-        COMPAS_FISP_CASE(17, 1)
-        COMPAS_FISP_CASE(18, 1)
-        COMPAS_FISP_CASE(19, 1)
-        COMPAS_FISP_CASE(20, 1)
-        COMPAS_FISP_CASE(21, 1)
-        COMPAS_FISP_CASE(22, 1)
-        COMPAS_FISP_CASE(23, 1)
-        COMPAS_FISP_CASE(24, 1)
-        COMPAS_FISP_CASE(25, 1)
-        COMPAS_FISP_CASE(26, 1)
-        COMPAS_FISP_CASE(27, 1)
-        COMPAS_FISP_CASE(28, 1)
-        COMPAS_FISP_CASE(29, 1)
-        COMPAS_FISP_CASE(30, 1)
-        COMPAS_FISP_CASE(31, 1)
-        COMPAS_FISP_CASE(32, 1)
-        default:
-            return nullptr;
-    }
-}
-
-static FispLauncher fisp_launcher_lpv2(int spl) {
-    switch (spl) {
-        COMPAS_FISP_CASE(1, 2)
-        COMPAS_FISP_CASE(2, 2)
-        COMPAS_FISP_CASE(3, 2)
-        COMPAS_FISP_CASE(4, 2)
-        COMPAS_FISP_CASE(5, 2)
-        COMPAS_FISP_CASE(6, 2)
-        COMPAS_FISP_CASE(7, 2)
-        COMPAS_FISP_CASE(8, 2)
-        COMPAS_FISP_CASE(9, 2)
-        COMPAS_FISP_CASE(10, 2)
-        COMPAS_FISP_CASE(11, 2)
-        COMPAS_FISP_CASE(12, 2)
-        COMPAS_FISP_CASE(13, 2)
-        COMPAS_FISP_CASE(14, 2)
-        COMPAS_FISP_CASE(15, 2)
-        COMPAS_FISP_CASE(16, 2)
-        COMPAS_FISP_CASE(32, 2)
-        default:
-            return nullptr;
-    }
-}
-
-static FispLauncher fisp_launcher_lpv4(int spl) {
-    switch (spl) {
-        COMPAS_FISP_CASE(1, 4)
-        COMPAS_FISP_CASE(2, 4)
-        COMPAS_FISP_CASE(3, 4)
-        COMPAS_FISP_CASE(4, 4)
-        COMPAS_FISP_CASE(5, 4)
-        COMPAS_FISP_CASE(6, 4)
-        COMPAS_FISP_CASE(7, 4)
-        COMPAS_FISP_CASE(8, 4)
-        COMPAS_FISP_CASE(32, 4)
-        default:
-            return nullptr;
-    }
-}
 
 Array<float4, 1> fisp_rf_table(const CompasContext& ctx, const FISPSequence& seq) {
     const int nTR = int(seq.RF_train.size(0)), nslices = int(seq.sliceprofiles.size(0));
@@ -194,34 +95,22 @@ int simd_count(int device) {
     return n;
 }
 
-// Lanes per voxel: pick the split with the lowest modelled time,
-// ceil(waves / SIMDs) * per-wave cost, cost ~ 26 VALU ops per local state per
-// TR plus ~90 ops of per-TR matrix set-up (duplicated in each lane of a voxel).
-// A wave alone on its SIMD issues at about half the rate of two co-resident
-// ones (50176 voxels x 25 states back to back: 1.90 ms in one lane per voxel,
-// 1.45 ms in two), but in the simulate + signal loop the one-lane layout is
-// faster (2.00-2.03 against 2.03-2.10 ms per launch after the contraction,
-// 2.30 against 2.43 ms per pipelined step): the model keeps one lane there.
+// Lanes per voxel and states per lane of the complex form: the lowest modelled
+// time of a TR.  A wave alone on its SIMD is bound by its chain of operations,
+// several by the instructions issued.  Constants (in us per TR) fitted to, in 1,
+// 2, 4 and 8 lanes: 1000 voxels x 25 states 1.34, 0.88, 0.51, 0.39; 50176 x 25
+// 1.38, 1.14, 1.25, 1.51; 200000 x 25 3.21, 3.38, 3.76, 4.88; 50176 x 60 -, 1.70,
+// 2.00, 2.20.  With 37 states 20011 voxels take 0.79 in four lanes of ten (1.79 in
+// two of 32, the only layout before for 33 to 64 states), 5000 x 60 0.62 in eight
+// (1.72).
 static void choose_fisp_layout(int N, int nvoxels, int simds, int* spl, int* lpv) {
-    if (N > 64) {
-        *spl = 32;
-        *lpv = 4;
-        return;
-    }
-    if (N > 32) {
-        *spl = 32;
-        *lpv = 2;
-        return;
-    }
     double best = 1e300;
-    for (int l : {1, 2, 4}) {
-        int s = (N + l - 1) / l;
-        if (l == 2 && s > 16) continue;
-        if (l == 4 && s > 8) continue;
-        const double waves = double(nvoxels) * l / 64.0;
-        const double rounds = std::ceil(waves / simds);
-        const double cost = rounds * (26.0 * s + 90.0 + (l > 1 ? 12.0 : 0.0));
-        if (cost < best - 1e-9) {
+    for (int l : {1, 2, 4, 8}) {
+        const int s = (N + l - 1) / l;
+        if (!fisp_epg_launcher(l, s)) continue;
+        const double waves = double(nvoxels) * l / 64.0 / simds;
+        const double cost = std::max(0.24 + 0.043 * s, 0.25 + waves * (0.045 + 0.0375 * s));
+        if (cost < best) {
             best = cost;
             *spl = s;
             *lpv = l;
@@ -355,15 +244,15 @@ static void launch_fisp_epg(
 
     int spl = 0, lpv = 0;
     choose_fisp_layout(seq.max_state, nv, simd_count(ctx.device()), &spl, &lpv);
-    if (const char* e = std::getenv("COMPAS_FISP_LPV")) {  // layout override (1, 2 or 4 lanes per voxel)
+    if (const char* e = std::getenv("COMPAS_FISP_LPV")) {  // layout override (1, 2, 4 or 8 lanes per voxel)
         const int l = std::atoi(e);
-        const int s = (seq.max_state + l - 1) / l;
-        if ((l == 1 && s <= 32) || (l == 2 && (s <= 16 || s == 32)) || (l == 4 && (s <= 8 || s == 32))) {
-            spl = (l > 1 && s > (l == 2 ? 16 : 8)) ? 32 : s;
+        const int s = l > 0 ? (seq.max_state + l - 1) / l : 0;
+        if (fisp_epg_launcher(l, s)) {
+            spl = s;
             lpv = l;
         }
     }
-    FispLauncher fn = lpv == 1 ? fisp_launcher_lpv1(spl) : lpv == 2 ? fisp_launcher_lpv2(spl) : fisp_launcher_lpv4(spl);
+    const FispLauncher fn = fisp_epg_launcher(lpv, spl);
     COMPAS_CHECK(fn != nullptr);
     unsigned blocks = dev::div_ceil(int64_t(nv) * lpv, 64);
     // both forms are launched, and the one that does not suit the train leaves
