@@ -55,8 +55,11 @@ def algorithmic_work(kernel: str, wl, method: str):
     nr, ns = wl.trajectory.nreadouts, wl.trajectory.samples_per_readout
     nc = wl.coils.shape[0]
     if kernel == "fisp_epg":
-        # 82 N flop per voxel.TR (excite 54 N + two rotate_decay 14 N)
-        return 82.0 * wl.sequence.max_state * nv * nTR / 1e12, "TFLOP/s", "valu", PEAK_FP32_TFLOPS
+        # flop per voxel.TR: 12 N for the real form that trains of real pulses take (S, D, the
+        # mixed S' and z', D' folded into the new F+ and F-), 82 N for the complex one (excite
+        # 54 N + two rotate_decay 14 N)
+        per_state = 82.0 if np.any(np.imag(wl.sequence.RF) != 0) else 12.0
+        return per_state * wl.sequence.max_state * nv * nTR / 1e12, "TFLOP/s", "valu", PEAK_FP32_TFLOPS
     if kernel in ("contraction_fp32", "contraction_mfma"):
         flops = 8.0 * nc * nr * ns * nv / 1e12
         if kernel == "contraction_mfma":
@@ -361,29 +364,27 @@ def spiral_bench(args):
     timings = ctx.read_kernel_timings()
     kernels = {k: {"launches": c, "avg_ms": tot / max(c, 1), "total_ms": tot} for k, (c, tot) in timings.items()}
 
-    # algorithmic work per launch: pSSFP (57 nRF + 28) flop per isochromat.TR (FP64 state); spiral
-    # sums 8 nc flop per (readout, sample, voxel) for the coil MACs + 6 for the sample recurrence
-    # (J.v: two amplitudes, 16 nc + 6); J^H.y: 8 nc (y conj(Phi)) + 8 nc (the (s - ns/2) moment) + 6.
-    # The spiral kernels run the contraction on MFMA (BF16 hi + lo: three v_mfma_f32_16x16x32_bf16
-    # per 16 voxels x 16 samples x 16 rows) and generate the sample factor on VALU, which binds:
-    # each entry gives the algorithmic rate against the FP32 vector peak and the issued MFMA
-    # fraction.
+    # algorithmic work: pSSFP maps, per isochromat.TR twelve polynomials of degree 7 and their
+    # application, 96 FMA (FP64). Spiral sums 8 nc flop per (readout, sample, voxel) for the coil
+    # MACs, 16 nc for J.v's two amplitudes, and for J^H.y's two moments. They run on MFMA with
+    # BF16 hi + lo operands (three products); the sample factor is generated on VALU in two
+    # levels, a few elements per (readout, voxel). Each of their entries gives the algorithmic
+    # rate and the issued fraction of the MFMA peak.
     rsv = float(nr) * ns * nv
     rooflines = {}
-    if "pssfp_iso" in kernels:
-        ach = (57.0 * nRF + 28) * nz * nTR * nv / (kernels["pssfp_iso"]["avg_ms"] * 1e-3) / 1e12
-        rooflines["pssfp_iso"] = {"bound": "valu", "achieved": ach, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-                                  "frac": ach / PEAK_FP64_TFLOPS,
-                                  "note": "FP64 isochromat state; the FP32 vector peak is twice this"}
-    issued = 2.0 * 16 * 2 * rsv * 3  # 16 real rows x 2 nv real K x ns x nr, three products
-    mfma_kernels = {"spiral_sum_mfma": ((8.0 * nc + 6) * rsv + (16.0 * nc + 6) * rsv, 2 * issued),  # signal + J.v
-                    "spiral_hermitian_mfma": ((16.0 * nc + 6) * rsv, issued)}
+    if "pssfp_map" in kernels:
+        ach = 192.0 * nz * nTR * nv / (kernels["pssfp_map"]["avg_ms"] * 1e-3) / 1e12
+        rooflines["pssfp_map"] = {"bound": "valu", "achieved": ach, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
+                                  "frac": ach / PEAK_FP64_TFLOPS}
+    issued = 8.0 * max(nc, 4) * rsv * 3  # coil rows x complex K x samples, three products
+    mfma_kernels = {"spiral_sum_mfma": (24.0 * nc * rsv, 3 * issued),  # signal + J.v
+                    "spiral_hermitian_mfma": (16.0 * nc * rsv, 2 * issued)}
     for k, (flop, iss) in mfma_kernels.items():
         if k in kernels:
             step_s = kernels[k]["total_ms"] / args.steps * 1e-3
             ach = flop / step_s / 1e12
-            rooflines[k] = {"bound": "valu", "achieved": ach, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-                            "frac": ach / PEAK_FP32_TFLOPS,
+            rooflines[k] = {"bound": "mfma", "achieved": ach, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
+                            "frac": ach / PEAK_BF16_TFLOPS,
                             "mfma_issued_frac": iss / step_s / 1e12 / PEAK_BF16_TFLOPS}
     for k, flop in (("signal_spiral_direct", (8.0 * nc + 6) * rsv + (16.0 * nc + 6) * rsv),
                     ("spiral_hermitian", (16.0 * nc + 6) * rsv)):
