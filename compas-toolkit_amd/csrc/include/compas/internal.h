@@ -98,8 +98,8 @@ void spiral_sum(
     int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out);
 
 // The same sums with the voxel contraction on MFMA (BF16 hi + lo, or hi only);
-// false when the precision is FP32 or the coils exceed one 16-row group
-// (eight with one amplitude, four with two): the caller runs the VALU form.
+// false when the precision is FP32 or there are more than eight coils with one
+// amplitude or four with two: the caller runs the VALU form.
 bool spiral_sum_mfma(
     const CompasContext& ctx, const TissueParameters& p, const cfloat* A, const cfloat* Ab, const cfloat* coils,
     int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out);

@@ -4,7 +4,10 @@
 // the EPG operators of src/operators/epg.cuh:19-322 (see the oracle for the
 // literal restatement).
 //
-// Design (MI355X):
+// A train of real pulses takes the real recursion (fisp_real.h); both kernels
+// are launched and one leaves at once.
+//
+// Design of the complex form (MI355X):
 //   * One voxel per lane (or LPV lanes per voxel for large state counts or
 //     small voxel counts).  The F+/F-/Z states of a voxel live in VGPRs; the
 //     dephasing shift is a register rename inside the unrolled update.
@@ -12,8 +15,9 @@
 //     regrow" is one real 3x3 matrix M = D(TR) R(alpha, phi) acting on the
 //     state written in the real transverse basis X = (F+ + F-)/2,
 //     Y = (F+ - F-)/(2i): 18 FMAs per state instead of ~40 for the complex
-//     F+/F-/Z form; the basis change costs 8 adds.  The TE sample F+_0(TE) uses
-//     the first two rows of D(TE) R on state 0 only.
+//     F+/F-/Z form; the basis change costs 8 adds.  The TE sample F+_0(TE) is
+//     the updated state 0 over the decay after TE (fisp_direct_echo: from the
+//     first two rows of D(TE) R where that decay underflows).
 //   * The RF table (alpha per unit B1, cos phi, sin phi) is precomputed per
 //     (slice, TR) and read with wave-uniform (scalar) loads.
 //   * Echoes are written directly in [nreadouts][nvoxels] layout (coalesced

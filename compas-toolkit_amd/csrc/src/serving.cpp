@@ -11,7 +11,7 @@
 //   2. Work-table launches.  Each launch takes up to batch_items() work items
 //      (a wave, or a workgroup of the pSSFP maps) from the active jobs, least GPU time used first (each
 //      job's virtual time grows by its item cost), groups them by kernel
-//      instance and launches fisp_epg_table / pssfp_iso_table over a table
+//      instance and launches fisp_epg_table, pssfp_map or pssfp_iso_table over a table
 //      uploaded from pinned memory.  Launches alternate over two streams with
 //      at most two in flight.  When a job's last item is launched, its
 //      completion step is enqueued on sim_[0] (after the other stream's
