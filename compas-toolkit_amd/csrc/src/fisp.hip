@@ -100,20 +100,23 @@ int simd_count(int device) {
 }
 
 // Lanes per voxel and states per lane of the complex form: the lowest modelled
-// time of a TR.  A wave alone on its SIMD is bound by its chain of operations,
-// several by the instructions issued.  Constants (in us per TR) fitted to, in 1,
-// 2, 4 and 8 lanes: 1000 voxels x 25 states 1.34, 0.88, 0.51, 0.39; 50176 x 25
-// 1.38, 1.14, 1.25, 1.51; 200000 x 25 3.21, 3.38, 3.76, 4.88; 50176 x 60 -, 1.70,
-// 2.00, 2.20.  With 37 states 20011 voxels take 0.79 in four lanes of ten (1.79 in
-// two of 32, the only layout before for 33 to 64 states), 5000 x 60 0.62 in eight
-// (1.72).
+// time of a TR, in us, of k = ceil(waves / SIMDs) waves sharing a SIMD with s
+// states per lane.  A wave alone is bound by its chain of operations, which a
+// second one fits beside; from then on the instructions issued count, and an
+// odd wave costs nearly a pair.  Measured and modelled, in 1, 2, 4 and 8 lanes:
+// 28701 voxels x 16 states 0.93 0.93, 0.58 0.58, 0.45 0.46, 0.62 0.61; 50176 x
+// 25 1.35 1.32, 0.88 0.87, 1.13 1.15, 1.39 1.56; 20011 x 37 -, 1.13 1.06, 0.79
+// 0.74, 0.87 0.93; 200000 x 25 3.21 3.10, 3.38 3.65.  With 37 states 20011 voxels
+// take 0.79 in four lanes of ten (1.79 in two of 32, the only layout before for
+// 33 to 64 states), 5000 x 60 0.62 in eight (1.72).
 static void choose_fisp_layout(int N, int nvoxels, int simds, int* spl, int* lpv) {
     double best = 1e300;
     for (int l : {1, 2, 4, 8}) {
         const int s = (N + l - 1) / l;
         if (!fisp_epg_launcher(l, s)) continue;
-        const double waves = double(nvoxels) * l / 64.0 / simds;
-        const double cost = std::max(0.24 + 0.043 * s, 0.25 + waves * (0.045 + 0.0375 * s));
+        double k = std::ceil(double(nvoxels) * l / 64.0 / simds);
+        if (k > 2.0) k = 2.0 * std::ceil(0.5 * k);
+        const double cost = std::max(0.24 + 0.043 * s, 0.15 + 0.06 * k + s * (0.031 * k - 0.0155));
         if (cost < best) {
             best = cost;
             *spl = s;
