@@ -418,7 +418,7 @@ Array<cfloat, 2> simulate_magnetization(
     // as one launch
     if (pssfp_map_pays(nTR, a.nRF) && L.groups <= L.per_launch) {
         auto train = ctx.empty<double, 1>({pssfp_map_train_size(nTR)});
-        kernels::PssfpMapArgs p;
+        kernels::PssfpMapArgs p {};
         pssfp_map_setup(ctx, p, a, train.data(), L.zpl);
         Array<cfloat, 2> part;
         if (const int planes = pssfp_map_partial_planes(p)) part = ctx.empty<cfloat, 2>({planes, plane});

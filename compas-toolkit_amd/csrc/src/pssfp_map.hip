@@ -35,6 +35,7 @@
 #include "compas/device/pssfp_common.h"
 #include "compas/device/pssfp_map.h"
 #include "compas/internal.h"
+#include "compas/pssfp_layout.h"
 
 namespace compas {
 namespace kernels {
@@ -335,25 +336,6 @@ __global__ void pssfp_map_sum(cfloat* __restrict__ echos, const cfloat* __restri
 
 }  // namespace kernels
 
-// Workgroup layout for nz slice positions: groups of equal size such that the
-// most of the 256 lanes hold an isochromat; a group after the first costs a
-// plane of partial echoes, so it has to raise that share by a tenth.
-static void map_layout(int nz, int* nv_block, int* nz_group, int* groups) {
-    double best = -1.0;
-    for (int g = (nz + 127) / 128, last = g + 4; g <= last && g <= nz; g++) {
-        const int zg = (nz + g - 1) / g;
-        if ((nz + zg - 1) / zg != g) continue;
-        const int vb = 256 / zg;
-        const double share = double(vb) * nz / g / 256.0 - 0.1 * g;
-        if (share > best) {
-            best = share;
-            *nv_block = vb;
-            *nz_group = zg;
-            *groups = g;
-        }
-    }
-}
-
 // Whether the maps pay for a train: per isochromat the sub-steps cost about
 // 31 nRF + 16 FP64 operations in every TR, the maps 100 and their set-up 80
 // nRF at each node.  Measured at 50176 voxels x 35 positions x 25 sub-steps:
@@ -380,7 +362,13 @@ void pssfp_map_setup(const CompasContext& ctx, kernels::PssfpMapArgs& p, const k
     p.a = a;
     p.train = train;
     p.partial = nullptr;
-    map_layout(a.nz, &p.nv_block, &p.nz_group, &p.groups);
+    // at least two voxels to a workgroup; a further group has to raise the lanes
+    // in use by a tenth
+    const PssfpWorkgroup w = pssfp_workgroup(a.nz, 256, 128, 0.1);
+    COMPAS_CHECK(w.groups > 0);
+    p.nv_block = w.nv_block;
+    p.nz_group = w.nz_group;
+    p.groups = w.groups;
     p.vblocks = int(dev::div_ceil(a.tissue.nvoxels, p.nv_block));
     p.direct_zpl = zpl;
     p.direct_groups = (a.nz + zpl - 1) / zpl;

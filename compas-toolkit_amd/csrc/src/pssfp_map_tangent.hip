@@ -31,6 +31,7 @@
 #include "compas/device/pssfp_map.h"
 #include "compas/device/tangent_set.h"
 #include "compas/internal.h"
+#include "compas/pssfp_layout.h"
 
 namespace compas {
 namespace kernels {
@@ -479,26 +480,6 @@ namespace {
 
 using namespace kernels;
 
-// Voxels and slice positions of a workgroup of `isos` isochromats; a further
-// group costs planes of partial sums, so it has to raise the lanes in use by a
-// twenty-fifth
-void tangent_layout(int nz, int isos, int* nv_block, int* nz_group, int* groups) {
-    double best = -1e9;
-    const int least = (nz + isos - 1) / isos;
-    for (int g = least; g <= least + 5 && g <= nz; g++) {
-        const int zg = (nz + g - 1) / g;
-        if ((nz + zg - 1) / zg != g) continue;
-        const int vb = isos / zg;
-        const double share = double(vb) * nz / g / isos - 0.04 * g;
-        if (share > best) {
-            best = share;
-            *nv_block = vb;
-            *nz_group = zg;
-            *groups = g;
-        }
-    }
-}
-
 template<int MASK>
 void run_pass(const CompasContext& ctx, const PssfpArgs& a, const double* train, cfloat* const* planes) {
     constexpr int NT = TangentSet<MASK>::nt, NP = TangentSet<MASK>::planes;
@@ -506,7 +487,12 @@ void run_pass(const CompasContext& ctx, const PssfpArgs& a, const double* train,
     t.p.a = a;
     t.p.train = train;
     for (int k = 0; k < NP; k++) t.out[k] = planes[k];
-    tangent_layout(a.nz, 128 / NT, &t.p.nv_block, &t.p.nz_group, &t.p.groups);
+    // a further group has to raise the isochromats in use by a twenty-fifth
+    const PssfpWorkgroup w = pssfp_workgroup(a.nz, 128 / NT, 128 / NT, 0.04);
+    COMPAS_CHECK(w.groups > 0);
+    t.p.nv_block = w.nv_block;
+    t.p.nz_group = w.nz_group;
+    t.p.groups = w.groups;
     const int64_t plane = int64_t(a.nTR) * a.tissue.nvoxels;
     Array<cfloat, 2> part;
     if (t.p.groups > 1) part = ctx.empty<cfloat, 2>({int64_t(t.p.groups - 1) * NP, plane});

@@ -86,3 +86,30 @@ def test_pssfp_map_tangents(oracle, fields, nv, nTR, nz, nRF, deg, phase):
     assert rel(out[0], oracle.pssfp(t, seq, "f64")) < TOL
     for f, d in zip(fields, out[1:]):
         assert rel(d, central_difference(oracle.pssfp, t, seq, ["T1", "T2", "B1", "B0"][f])) < 1e-6
+
+
+def test_many_slice_positions(oracle):
+    """2500 slice positions, 20 groups of them to a voxel block: the echoes, the
+    tangents and the request server.  Twenty FP32 partial planes and the echo's
+    own rounding, each 6e-8 of a part of the sum, and up to 2500 positions that
+    dephase by a radian: 1e-6; tangents as above with forty planes, 2e-6."""
+    banner("pssfp map 2500 slice positions")
+    context()
+    t = W.make_tissue(W.SplitMix64(77), 2, 20.0, 40.0).slice(0, 3)
+    seq = train(66, 45.0, 2500, 12, 0.6)
+    p, s = ca.TissueParameters.from_tissue(t), ca.pSSFPSequence.from_sequence(seq)
+    want = oracle.pssfp(t, seq, "f64")
+    got = ca.simulate_magnetization(p, s).collect()
+    assert rel(got, want) < 1e-6
+    out = [a.collect() for a in ca.simulate_magnetization_tangents((ca.T1, ca.T2), p, s, echos=True)]
+    assert rel(out[0], want) < 1e-6
+    for name, d in zip(("T1", "T2"), out[1:]):
+        assert rel(d, central_difference(oracle.pssfp, t, seq, name)) < 2e-6
+    traj = ca.SpiralTrajectory.from_trajectory(W.make_spiral(66, 32, 20.0, 8, 5e-6))
+    coils = ca.CompasArray.from_numpy(np.ones((1, 3), np.complex64))
+    server = ca.Server(slots=1, memory_budget=1 << 30)
+    ticket = server.submit_simulate_signal(p, s, traj, coils)
+    assert server.wait(ticket, timeout=60) is not None
+    assert np.array_equal(server.result(ticket, 0).collect(), got)
+    server.release(ticket)
+    server.close()
