@@ -6,10 +6,11 @@
 // (jacobian_spiral.hip states Phi and how U, U' combine into the six rows).
 // Phi is a geometric sequence in s: with s = sb + S t + n, n < S = 8 KS, Phi_s =
 // Phi_sb E^(S t) E^n and
-//   U  = conj(Phi_sb) sum_t conj(E^(S t)) G_t,   G_t  = sum_n y_(sb + S t + n) conj(E^n)
-//   U' = conj(Phi_sb) sum_t conj(E^(S t)) ((sb + S t - ns/2) G_t + G'_t),
-//                                              G'_t = sum_n n y_(sb + S t + n) conj(E^n).
-// G and G' are a complex GEMM, rows (coil, t) x K = n x N = voxels, whose B
+//   U  = conj(Phi_sb) sum_t conj(E^(S t)) G_t,   G_t  = sum_n y_s conj(E^n)
+//   U' = conj(Phi_sb) sum_t conj(E^(S t)) G'_t,  G'_t = sum_n (s - ns/2) y_s conj(E^n).
+// (s - ns/2 in one piece: split as (sb + S t - ns/2) G_t + sum_n n y_s conj(E^n) its
+// two terms cancel near the centre of the readout, where a readout peaks, after
+// each has been rounded.)  G and G' are a complex GEMM, rows (coil, t) x K = n x N = voxels, whose B
 // operand has S generated elements per voxel and readout instead of ns; the
 // sums over t are Horner's rule on the accumulators.  It runs on
 // v_mfma_f32_32x32x16_bf16 with BF16 hi + lo operands (FP32 accumulation):
@@ -78,7 +79,7 @@ __global__ void __launch_bounds__(64 * KS) spiral_y_fragments(
     for (int j = 0; j < 4; j++) {
         cfloat v = {0.0f, 0.0f};
         if (c < nc && s0 + j < ns) v = y[(size_t(c) * nr + r) * ns + s0 + j];
-        const cfloat w = v * float(n0 + j);
+        const cfloat w = v * (float(s0 + j) - 0.5f * float(ns));
         mfma::split_pair<P>(v.re, v.im, hi[0][j], lo[0][j]);
         mfma::split_pair<P>(v.im, -v.re, hi[1][j], lo[1][j]);
         mfma::split_pair<P>(w.re, w.im, hi[2][j], lo[2][j]);
@@ -221,9 +222,8 @@ __global__ void __launch_bounds__(64 * W, W / 4) spiral_hermitian_mfma(
 #pragma unroll
                     for (int t = NT - 1; t >= 0; t--) {
                         const int e = NT * k + t;
-                        const float tau = float(sb + S * t) - 0.5f * float(ns);
                         const cfloat G = {acc[i][0][e], acc[i][1][e]};
-                        const cfloat H = {fmaf(tau, G.re, acc[i][2][e]), fmaf(tau, G.im, acc[i][3][e])};
+                        const cfloat H = {acc[i][2][e], acc[i][3][e]};
                         U = t == NT - 1 ? G : dev::cfma_conj(U, eS[i], G);
                         Up = t == NT - 1 ? H : dev::cfma_conj(Up, eS[i], H);
                     }

@@ -1,0 +1,49 @@
+"""Accuracy of the spiral products where one part of them stands alone: the
+(s - ns/2) moment, and sums over many readouts."""
+
+import numpy as np
+import pytest
+
+import compas_amd as ca
+from compas_amd import workloads as W
+from gpu_helpers import banner, context, rel
+
+pytestmark = pytest.mark.gpu
+
+
+def objects(nv, nr, ns, nc):
+    n = int(np.ceil(np.sqrt(nv)))
+    t = W.make_tissue(W.SplitMix64(8), n, 20.0, 40.0).slice(0, nv)
+    traj = W.make_spiral(nr, ns, 20.0, max(n, 8), 5e-6)
+    coils = W.make_coils(n, 20.0, nc)[:, :nv]
+    context()
+    return t, traj, coils, ca.TissueParameters.from_tissue(t), ca.SpiralTrajectory.from_trajectory(traj)
+
+
+def noise(rng, *shape):
+    return (rng.normal(size=shape) + 1j * rng.normal(size=shape)).astype(np.complex64)
+
+
+# a BF16 hi + lo pair keeps a number to 2^-18 and the product of the two lo parts
+# is dropped, 3 x 3.8e-6 of a term; one BF16 product keeps 2^-9 of each operand
+METHODS = [("gemm_fast", 1.2e-5), ("gemm_low", 4e-3)]
+
+
+@pytest.mark.parametrize("ns", [31, 64, 130, 250, 500, 512, 1040])
+@pytest.mark.parametrize("width", [5.0, 20.0])
+@pytest.mark.parametrize("method,tol", METHODS)
+def test_adjoint_moment_of_a_peaked_readout(oracle, ns, width, method, tol):
+    """Readouts that peak where they cross the centre of k-space, s = ns/2; with
+    zero derivatives the T2 and B0 rows of J^H.y are the moment alone."""
+    banner(f"spiral J^H.y moment {ns} samples, window {width}, {method}")
+    nv, nr, nc = 130, 3, 4
+    t, traj, coils, p, tr = objects(nv, nr, ns, nc)
+    rng = np.random.default_rng(ns)
+    m = noise(rng, nr, nv)
+    zero = [np.zeros((nr, nv), np.complex64)] * 4
+    y = noise(rng, nc, nr, ns) * np.exp(-0.5 * ((np.arange(ns) - ns / 2) / width) ** 2).astype(np.float32)
+    wide = lambda a: a.astype(np.complex128)  # noqa: E731
+    want = oracle.jacobian_hermitian_spiral(t, traj, coils, wide(m), *[wide(z) for z in zero], wide(y), "f64")
+    got = ca.compute_jacobian_hermitian_spiral(m, zero, p, tr, coils, y, method=method).collect()
+    for row in (1, 3):
+        assert rel(got[row], want[row]) < tol
