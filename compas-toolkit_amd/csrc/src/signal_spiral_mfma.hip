@@ -6,9 +6,10 @@
 // is a complex GEMM with rows (coil, t), columns n < S and K = voxels: A = C A_r
 // E^(sb + S t), B = E^n.  Per voxel and readout nc T + S elements are generated
 // instead of one for every sample (96 instead of 512 at 4 coils x 512
-// samples), for the same MFMA products.  Of the two amplitudes, (s - ns/2) Ab =
-// (sb + S t - ns/2) Ab + n Ab: the first term joins A's rows, the second has
-// rows of its own, whose sum the epilogue multiplies by n.
+// samples), for the same MFMA products.  Of two amplitudes each has rows of its
+// own; the pass that adds the voxel ranges multiplies the second sum by s - ns/2
+// (taken apart into sb + S t - ns/2 and n, its two terms would cancel near the
+// centre of the readout after each was rounded).
 //
 // A wave owns a readout and a voxel range and walks it eight voxels at a time
 // (one K step of v_mfma_f32_32x32x16_bf16):
@@ -82,9 +83,9 @@ __global__ void spiral_voxels(dev::TissueView t, float dt, SpiralVoxel* __restri
     out[v] = o;
 }
 
-// grid (nr, voxel ranges, sample passes), block 64
 typedef float f32x16s __attribute__((ext_vector_type(16)));
 
+// grid (nr, voxel ranges, sample passes), block 64
 template<int CT, int RT, bool TWO, bool LO>
 __global__ void __launch_bounds__(64, 2) spiral_sum_split(
     const SpiralVoxel* __restrict__ voxels, int nv, const cfloat* __restrict__ A, const cfloat* __restrict__ Ab,
@@ -123,7 +124,6 @@ __global__ void __launch_bounds__(64, 2) spiral_sum_split(
                 for (int e = 0; e < 16; e++) acc[i][k][j][e] = 0.0f;
 
     const float s_amp = float(sb + S * q);  // the slot's sample
-    const float tau = s_amp - 0.5f * float(ns);
     // the next step's voxel is loaded a step ahead
     SpiralVoxel nx;
     cfloat na, nb {};
@@ -150,14 +150,11 @@ __global__ void __launch_bounds__(64, 2) spiral_sum_split(
         cfloat e8 = {__shfl(ph.re, 32 + gv), __shfl(ph.im, 32 + gv)};
         e8 = dev::cmul(e8, e8);
         const cfloat w = spiral_phasor(s_amp * x.decay, double(s_amp) * turns);
+        const cfloat u = dev::cmul(a, w);
+        amp[0][lane] = make_float2(u.re, u.im);
         if constexpr (TWO) {
-            const cfloat u = dev::cmul(cfloat {fmaf(tau, ab.re, a.re), fmaf(tau, ab.im, a.im)}, w);
             const cfloat ub = dev::cmul(ab, w);
-            amp[0][lane] = make_float2(u.re, u.im);
             amp[1][lane] = make_float2(ub.re, ub.im);
-        } else {
-            const cfloat u = dev::cmul(a, w);
-            amp[0][lane] = make_float2(u.re, u.im);
         }
 #pragma unroll
         for (int m = 0; m < S / 8; m++) {
@@ -198,7 +195,9 @@ __global__ void __launch_bounds__(64, 2) spiral_sum_split(
         __syncthreads();
     }
 
-    cfloat* base = partial + size_t(blockIdx.y) * (size_t(nc) * nr * ns);
+    // with two amplitudes a plane for each
+    const size_t plane = size_t(nc) * nr * ns;
+    cfloat* base = partial + size_t(blockIdx.y) * (TWO ? 2 : 1) * plane;
 #pragma unroll
     for (int i = 0; i < (TWO ? 1 : RT); i++)
 #pragma unroll
@@ -209,25 +208,36 @@ __global__ void __launch_bounds__(64, 2) spiral_sum_split(
             for (int j = 0; j < CT; j++) {
                 const int n = 32 * j + col, s = sb + S * tt + n;
                 if (c < nc && s < ns) {
-                    cfloat o = {acc[i][0][j][e], acc[i][1][j][e]};
-                    if constexpr (TWO) {
-                        o.re = fmaf(float(n), acc[RT - 1][0][j][e], o.re);
-                        o.im = fmaf(float(n), acc[RT - 1][1][j][e], o.im);
-                    }
-                    base[(size_t(c) * nr + r) * ns + s] = o;
+                    const size_t o = (size_t(c) * nr + r) * ns + s;
+                    base[o] = {acc[i][0][j][e], acc[i][1][j][e]};
+                    if constexpr (TWO) base[plane + o] = {acc[RT - 1][0][j][e], acc[RT - 1][1][j][e]};
                 }
             }
         }
 }
 
-// out[i] = sum over the splits (FP64, in order)
-__global__ void spiral_sum_reduce(const cfloat* __restrict__ partial, int splits, int64_t n, cfloat* __restrict__ out) {
+// out[i] = sum over the splits (FP64, in order); with two amplitudes out =
+// first + (s - ns/2) second, s = i % ns
+template<bool TWO>
+__global__ void spiral_sum_reduce(
+    const cfloat* __restrict__ partial, int splits, int64_t n, int ns, cfloat* __restrict__ out) {
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
-        double re = 0.0, im = 0.0;
+        double re = 0.0, im = 0.0, bre = 0.0, bim = 0.0;
         for (int k = 0; k < splits; k++) {
-            const cfloat p = partial[size_t(k) * size_t(n) + size_t(i)];
+            const size_t o = size_t(k) * (TWO ? 2 : 1) * size_t(n) + size_t(i);
+            const cfloat p = partial[o];
             re += p.re;
             im += p.im;
+            if constexpr (TWO) {
+                const cfloat q = partial[o + size_t(n)];
+                bre += q.re;
+                bim += q.im;
+            }
+        }
+        if constexpr (TWO) {
+            const double sp = double(i % ns) - 0.5 * double(ns);
+            re = fma(sp, bre, re);
+            im = fma(sp, bim, im);
         }
         out[i] = {float(re), float(im)};
     }
@@ -267,7 +277,7 @@ bool spiral_sum_mfma(
     const int v_chunk = int(dev::div_ceil(dev::div_ceil(nv, splits0), 8)) * 8;
     const int splits = int(dev::div_ceil(nv, v_chunk));
     const int64_t plane = int64_t(nc) * nr * ns;
-    auto partial = ctx.empty<cfloat, 1>({int64_t(splits) * plane});
+    auto partial = ctx.empty<cfloat, 1>({int64_t(splits) * (two ? 2 : 1) * plane});
     auto voxels = spiral_voxel_table(ctx, p, t.delta_t);
     {
         KernelScope ks(ctx, "spiral_sum_mfma");
@@ -292,7 +302,8 @@ bool spiral_sum_mfma(
     }
     KernelScope ks(ctx, "spiral_sum_reduce");
     const int64_t blocks = std::min<int64_t>(dev::div_ceil(plane, int64_t(256)), 8192);
-    kernels::spiral_sum_reduce<<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, out);
+    if (two) kernels::spiral_sum_reduce<true><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
+    else kernels::spiral_sum_reduce<false><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
     check_launch("spiral_sum_reduce");
     return true;
 }

@@ -47,3 +47,23 @@ def test_adjoint_moment_of_a_peaked_readout(oracle, ns, width, method, tol):
     got = ca.compute_jacobian_hermitian_spiral(m, zero, p, tr, coils, y, method=method).collect()
     for row in (1, 3):
         assert rel(got[row], want[row]) < tol
+
+
+@pytest.mark.parametrize("ns", [31, 64, 130, 250, 500, 512, 1040])
+@pytest.mark.parametrize("method,tol", METHODS)
+def test_product_moment_at_the_centre(oracle, ns, method, tol):
+    """With zero derivatives a step in T2 and B0 changes the signal by s - ns/2
+    times a sum: the samples within four of ns/2, where that factor is small."""
+    banner(f"spiral J.v moment {ns} samples, {method}")
+    nv, nr, nc = 130, 3, 4
+    t, traj, coils, p, tr = objects(nv, nr, ns, nc)
+    rng = np.random.default_rng(ns + 1)
+    m = noise(rng, nr, nv)
+    zero = [np.zeros((nr, nv), np.complex64)] * 4
+    v = noise(rng, 6, nv)
+    v[[0, 2, 4, 5]] = 0
+    wide = lambda a: a.astype(np.complex128)  # noqa: E731
+    want = oracle.jacobian_spiral(t, traj, coils, wide(m), *[wide(z) for z in zero], wide(v), "f64")
+    got = ca.compute_jacobian_spiral(m, zero, p, tr, coils, v, method=method).collect()
+    at = slice(max(0, ns // 2 - 4), ns // 2 + 5)
+    assert rel(got[..., at], want[..., at]) < tol
