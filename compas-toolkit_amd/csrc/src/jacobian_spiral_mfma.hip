@@ -307,7 +307,10 @@ bool spiral_hermitian_mfma(
             check_launch("spiral_y_fragments");
         }
         // readout chunks: the fewest rounds of resident workgroups times a chunk's
-        // readouts (and two readouts' worth of beginning and end)
+        // readouts (and two readouts' worth of beginning and end).  A chunk is summed
+        // in FP32 and the chunks in FP64, so a chunk is no longer than 192 readouts
+        // (98304 voxels x 1120 readouts in one chunk: 4.9e-7 of a constant sum, in
+        // six 8e-8)
         static const int resident = [] {
             int n = 0;
             COMPAS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
@@ -317,7 +320,8 @@ bool spiral_hermitian_mfma(
         const int64_t slots = int64_t(simd_count(ctx.device()) / 4) * resident;
         int r_chunk = nr;
         int64_t best = INT64_MAX;
-        for (int n = 1; n <= nr && (n == 1 || int64_t(n) * vblocks <= 8 * slots); n++) {
+        const int fewest = int(dev::div_ceil(nr, 192));
+        for (int n = fewest; n <= nr && (n == fewest || int64_t(n) * vblocks <= 8 * slots); n++) {
             const int size = int(dev::div_ceil(nr, n));
             const int64_t cost = int64_t(dev::div_ceil(int64_t(dev::div_ceil(nr, size)) * vblocks, slots)) * (size + 2);
             if (cost < best) {

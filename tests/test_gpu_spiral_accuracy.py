@@ -67,3 +67,29 @@ def test_product_moment_at_the_centre(oracle, ns, method, tol):
     got = ca.compute_jacobian_spiral(m, zero, p, tr, coils, v, method=method).collect()
     at = slice(max(0, ns // 2 - 4), ns // 2 + 5)
     assert rel(got[..., at], want[..., at]) < tol
+
+
+def test_adjoint_over_many_readouts():
+    """1120 readouts of a constant field over as many voxels as the GPU takes in
+    one round of workgroups: a voxel's sum over the readouts is FP32 within a
+    chunk of readouts and FP64 over the chunks.  Every product is exact here, and a
+    chain of L additions leaves 2.5e-8 L / sqrt(3 x 1120) of the sum: 8.3e-8 at
+    192, and 2.5e-8 for the result."""
+    import torch
+
+    banner("spiral J^H.y over 1120 readouts")
+    context()
+    nv, nr, ns = 98304, 1120, 512
+    one, nil = np.ones(nv, np.float32), np.zeros(nv, np.float32)
+    p = ca.TissueParameters(nv, one, np.full(nv, 1e30, np.float32), one, nil, one, nil, nil, nil)
+    tr = ca.SpiralTrajectory(nr, ns, 5e-6, np.zeros(nr, np.complex64), np.zeros(nr, np.complex64))
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(3)
+    x = torch.rand(nr, nv, device="cuda:0", generator=gen) + 0.5
+    m = ca.CompasArray.from_dlpack(torch.complex(x, torch.zeros_like(x)))
+    coils = ca.CompasArray.from_numpy(np.ones((1, nv), np.complex64))
+    y = ca.CompasArray.from_numpy(np.ones((1, nr, ns), np.complex64))
+    got = ca.compute_jacobian_hermitian_spiral(m, [m] * 4, p, tr, coils, y, method="gemm_fast").collect()
+    want = ns * x.double().sum(0).cpu().numpy()
+    for row in (0, 4):
+        assert rel(got[row], want) < 1.5e-7
