@@ -174,6 +174,7 @@ void launch_pssfp_table(
 // the maps: that form and the sum of the partial planes.
 bool pssfp_map_pays(int nTR, int nRF);
 int64_t pssfp_map_train_size(int nTR);
+constexpr int pssfp_map_served_entry = 1;  // of the table: not 0 if the maps serve the train
 void pssfp_map_setup(const CompasContext& ctx, kernels::PssfpMapArgs& p, const kernels::PssfpArgs& a, double* train, int zpl);
 int pssfp_map_partial_planes(const kernels::PssfpMapArgs& p);
 int64_t pssfp_map_units(const kernels::PssfpMapArgs& p);

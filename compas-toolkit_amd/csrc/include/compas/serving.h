@@ -127,6 +127,7 @@ class Server {
     void post_process(Entry& e, int slot);  // the request's contraction after its simulations
     void admit(int64_t ticket, Entry& e);
     void activate_jobs(int64_t ticket, Entry& e);
+    void decide_jobs();
     void build_and_launch_batch();
     void complete_jobs();
     void fail_simulations(const std::string& error);  // every request of admitted_ ends with `error`
@@ -148,6 +149,8 @@ class Server {
     static constexpr size_t kRingBytes = size_t(1) << 20;
     void* host_ring_[kRing] = {};
     Array<uint8_t, 1> dev_ring_[kRing];
+    void* host_flags_ = nullptr;  // pinned: the answers to whether the maps serve a pSSFP train
+    std::vector<double*> free_flags_;
     std::shared_ptr<Event> ring_busy_[kRing];
     std::shared_ptr<Event> stream_busy_[kSimStreams];  // each stream's last launch
     hipEvent_t alloc_event_ = nullptr;  // recorded on sim_[0] after job memory is set up

@@ -27,7 +27,8 @@
 //     the set-up); the rest is the waits around the chunk sums.
 //   * Whether a train is within MAP_MAX_TYPE is found on the device: the train
 //     lives there and may be rewritten between calls.  The sub-step kernel is
-//     launched after this one, and one of the two leaves at once.
+//     launched after this one, and one of the two leaves at once (the request
+//     server reads the answer back and cuts the sub-steps into work items).
 
 #include <algorithm>
 

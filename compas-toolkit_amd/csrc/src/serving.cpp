@@ -7,12 +7,15 @@
 //      perturbed simulation per finite-difference field.  Job memory (echoes,
 //      FISP RF tables, pSSFP partial planes, perturbed tissue copies) comes
 //      from the pool of sim_[0], set up on its stream after the request's
-//      inputs are ready.
+//      inputs are ready.  Whether a pSSFP train is within the per-TR maps is
+//      found on the device: a job begins with the items of the maps, which
+//      leave at once where it is not, and gets those of the sub-step form
+//      instead when that answer has come back to pinned memory.
 //   2. Work-table launches.  Each launch takes up to batch_items() work items
-//      (a wave, or a workgroup of the pSSFP maps) from the active jobs, least GPU time used first (each
-//      job's virtual time grows by its item cost), groups them by kernel
-//      instance and launches fisp_epg_table, pssfp_map or pssfp_iso_table over a table
-//      uploaded from pinned memory.  Launches alternate over two streams with
+//      (a wave, or a workgroup of the pSSFP maps) from the active jobs, least
+//      GPU time used first (each job's virtual time grows by its item cost),
+//      groups them by kernel instance and launches fisp_epg_table, pssfp_map or
+//      pssfp_iso_table over a table uploaded from pinned memory.  Launches alternate over two streams with
 //      at most two in flight.  When a job's last item is launched, its
 //      completion step is enqueued on sim_[0] (after the other stream's
 //      launches that held its items): the pSSFP group sum, and for a
@@ -141,6 +144,8 @@ struct Server::SimJob {
     int field = -1;  // finite-difference field of this job, -1 for the echoes
     bool pssfp = false;
     bool maps = false;  // pSSFP by per-TR maps (pssfp_map.hip); an item is one of its units
+    std::shared_ptr<double> served;  // until the answer is read: pinned, not 0 if the maps serve the train
+    std::shared_ptr<Event> decided;  // when `served` holds it
     int bucket = 0;  // kernel instance: FISP states per lane, pSSFP slice positions per lane
     int vblocks = 0, groups = 1;
     int64_t items = 0, next = 0;  // work items, and the first not yet launched
@@ -159,9 +164,30 @@ struct Server::SimJob {
 namespace {
 std::atomic<uint64_t> g_next_server_id {1};
 
+// the partial planes and the work items of a pSSFP job, by maps or by sub-steps
+void make_items(const CompasContext& sim, Server::SimJob& j, bool maps) {
+    const kernels::PssfpArgs& a = j.pss.a;
+    j.maps = maps;
+    j.next = 0;
+    if (maps) {
+        j.groups = j.map.groups;
+        j.items = pssfp_map_units(j.map);
+        j.bucket = 0;  // one kernel instance for all
+        j.item_cost = 4.0 * (100.0 * a.nTR + 700.0 * a.nRF);
+    } else {
+        j.bucket = pssfp_table_zpl(a.nz);
+        j.groups = (a.nz + j.bucket - 1) / j.bucket;
+        j.items = int64_t(j.vblocks) * j.groups;
+        j.item_cost =
+            double(a.nTR + 1) * std::max(a.nRF, 1) * (j.bucket * 50.0 + 12.0) + double(a.nTR) * j.bucket * 40.0;
+    }
+    if (j.groups > 1) j.partial = sim.empty<cfloat, 2>({j.groups - 1, int64_t(a.nTR) * a.tissue.nvoxels});
+    j.map.partial = j.pss.partial = j.partial.data();
+}
+
 // the job's simulation set up on `sim` (its stream already ordered after the
-// request's inputs): output arrays, RF table or partial planes, the kernel
-// arguments and the work items
+// request's inputs): output arrays, RF table, the kernel arguments and the work
+// items
 std::shared_ptr<Server::SimJob> make_job(const CompasContext& sim, const ServeRequest& r, int64_t ticket, size_t k) {
     auto j = std::make_shared<Server::SimJob>();
     j->ticket = ticket;
@@ -209,11 +235,6 @@ std::shared_ptr<Server::SimJob> make_job(const CompasContext& sim, const ServeRe
         j->echos = sim.empty<cfloat, 2>({nTR, nv});
         if (nv > 0 && nz == 0) sim.fill_zero(j->echos.data(), j->echos.nbytes());
         if (nv > 0 && nz > 0) {
-            const int zpl = pssfp_table_zpl(nz);
-            j->bucket = zpl;
-            j->groups = (nz + zpl - 1) / zpl;
-            const int64_t plane = int64_t(nTR) * nv;
-            j->maps = pssfp_map_pays(nTR, nRF);
             kernels::PssfpArgs& a = j->pss.a;
             a.tissue = dev::tissue_view(j->params);
             a.RF = seq.RF_train.data();
@@ -228,20 +249,12 @@ std::shared_ptr<Server::SimJob> make_job(const CompasContext& sim, const ServeRe
             a.g_ex = seq.gamma_dt_GRz.ex;
             a.g_pr = seq.gamma_dt_GRz.pr;
             a.echos = j->echos.data();
-            if (j->maps) {
+            const bool maps = pssfp_map_pays(nTR, nRF);
+            if (maps) {
                 j->train = sim.empty<double, 1>({pssfp_map_train_size(nTR)});
-                pssfp_map_setup(sim, j->map, a, j->train.data(), zpl);
-                if (const int planes = pssfp_map_partial_planes(j->map)) j->partial = sim.empty<cfloat, 2>({planes, plane});
-                j->map.partial = j->partial.data();
-                j->items = pssfp_map_units(j->map);
-                j->bucket = 0;  // one kernel instance for all
-                j->item_cost = 4.0 * (100.0 * nTR + 700.0 * nRF);
-                return j;
+                pssfp_map_setup(sim, j->map, a, j->train.data(), pssfp_table_zpl(nz));
             }
-            if (j->groups > 1) j->partial = sim.empty<cfloat, 2>({j->groups - 1, plane});
-            j->pss.partial = j->partial.data();
-            j->items = int64_t(j->vblocks) * j->groups;
-            j->item_cost = double(nTR + 1) * std::max(nRF, 1) * (zpl * 50.0 + 12.0) + double(nTR) * zpl * 40.0;
+            make_items(sim, *j, maps);
         }
     }
     return j;
@@ -266,6 +279,9 @@ Server::Server(const CompasContext& base, int slots, size_t memory_budget) :
         rt->set_autotune(false);
         sim_.emplace_back(rt);
     }
+    // an admitted request waits for one answer at a time
+    COMPAS_HIP_CHECK(hipHostMalloc(&host_flags_, kMaxActive * sizeof(double), hipHostMallocDefault));
+    for (int i = 0; i < kMaxActive; i++) free_flags_.push_back(static_cast<double*>(host_flags_) + i);
     for (int r = 0; r < kRing; r++) {
         COMPAS_HIP_CHECK(hipHostMalloc(&host_ring_[r], kRingBytes, hipHostMallocDefault));
         dev_ring_[r] = sim_[0].empty<uint8_t, 1>({int64_t(kRingBytes)});
@@ -288,6 +304,7 @@ Server::~Server() {
     for (int r = 0; r < kRing; r++) {
         if (host_ring_[r]) (void)hipHostFree(host_ring_[r]);
     }
+    if (host_flags_) (void)hipHostFree(host_flags_);
     if (alloc_event_) (void)hipEventDestroy(alloc_event_);
 }
 
@@ -426,7 +443,37 @@ void Server::activate_jobs(int64_t ticket, Entry& e) {
             }
         }
         job->vtime = vmin;
+        if (job->maps) {  // ask whether they serve the train
+            COMPAS_CHECK(!free_flags_.empty());
+            double* flag = free_flags_.back();
+            free_flags_.pop_back();
+            job->served = std::shared_ptr<double>(flag, [this](double* f) { free_flags_.push_back(f); });
+            COMPAS_HIP_CHECK(hipMemcpyAsync(
+                flag, job->train.data() + pssfp_map_served_entry, sizeof(double), hipMemcpyDeviceToHost, sim.stream()));
+            job->decided = std::make_shared<Event>();
+            COMPAS_HIP_CHECK(hipEventRecord(job->decided->ev, sim.stream()));
+        }
         if (job->items > 0) active_jobs_.push_back(job);
+        any = true;
+    }
+    if (any) COMPAS_HIP_CHECK(hipEventRecord(alloc_event_, sim.stream()));
+}
+
+// Reads the device's answers: a pSSFP job whose train the maps do not serve
+// goes on with the items of the sub-step form.
+void Server::decide_jobs() {
+    const CompasContext& sim = sim_[0];
+    sim.activate();
+    bool any = false;
+    for (auto& j : active_jobs_) {
+        if (!j->served) continue;
+        const hipError_t q = hipEventQuery(j->decided->ev);
+        if (q == hipErrorNotReady) continue;
+        COMPAS_HIP_CHECK(q);
+        const bool maps = *j->served != 0.0;
+        j->served.reset();
+        if (maps) continue;
+        make_items(sim, *j, false);
         any = true;
     }
     if (any) COMPAS_HIP_CHECK(hipEventRecord(alloc_event_, sim.stream()));
@@ -454,14 +501,12 @@ void Server::complete_jobs() {
         bool progressed = false;
         for (size_t k = 0; k < e->next_job; k++) {
             SimJob& j = *e->jobs[k];
-            if (j.completed || j.next < j.items) continue;
+            if (j.completed || j.served || j.next < j.items) continue;
             if (k > 0 && !e->jobs[0]->completed) continue;
             for (int st = 1; st < kSimStreams; st++) {
                 if (j.last[st]) COMPAS_HIP_CHECK(hipStreamWaitEvent(sim.stream(), j.last[st]->ev, 0));
             }
-            if (j.maps) {
-                pssfp_map_finish(sim, j.map);
-            } else if (j.pssfp && j.groups > 1) {
+            if (j.pssfp && j.groups > 1) {
                 const int64_t plane = j.echos.numel();
                 pssfp_sum_groups(sim, j.echos.data(), j.partial.data(), j.groups - 1, plane, plane);
             }
@@ -766,6 +811,7 @@ void Server::dispatch_loop() {
         // requests whose simulations are not complete, and the server goes on
         try {
             for (int round = 0; round < 2; round++) {
+                decide_jobs();
                 complete_jobs();
                 build_and_launch_batch();
             }

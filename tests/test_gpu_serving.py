@@ -253,3 +253,57 @@ def test_inputs_still_queued_on_the_base_stream(i):
     server.close()
     want = run_alone((kind, p, s, tr, coils, res))
     assert np.array_equal(got, want)
+
+
+def test_pssfp_beyond_the_maps_is_cut_into_items():
+    """A pSSFP train too strong for the per-TR maps, or with a NaN among the B1
+    values, is known as such only on the device: its simulation still runs as work
+    items of the sub-step form, the larger one over several launches, and never as
+    one launch in the completion step; the results are those of the plain calls."""
+    banner("serving: pSSFP beyond the maps")
+    context()
+    nv, nTR, nz = 30016, 64, 35
+    t = W.make_tissue(W.SplitMix64(5), 174, 20.0, 40.0).slice(0, nv)
+    weak, strong = W.make_pssfp(nTR, 60.0, nz=nz, nRF=25), W.make_pssfp(nTR, 170.0, nz=nz, nRF=25)
+    small = W.make_tissue(W.SplitMix64(6), 30, 20.0, 40.0)
+    outlier = small.replace(B1=np.where(np.arange(900) == 17, np.nan, small.B1).astype(np.float32))
+    traj = ca.SpiralTrajectory.from_trajectory(W.make_spiral(nTR, 16, 20.0, 174, 5e-6))
+    # launches of sub-step items: 469 and 15 blocks of 64 voxels x 5 groups of
+    # positions, 2048 to a launch
+    cases = [(t, weak, 0), (t, strong, 2), (outlier, weak, 1)]
+    objs = [(ca.TissueParameters.from_tissue(a), ca.pSSFPSequence.from_sequence(b),
+             ca.CompasArray.from_numpy(np.ones((1, len(a.T1)), np.complex64))) for a, b, _ in cases]
+    server = ca.Server(slots=2, memory_budget=8 << 30)
+    server.set_kernel_timing(True)
+
+    def sub_step_launches():
+        timings = server.read_kernel_timings()
+        assert "pssfp_iso" not in timings
+        return timings.get("pssfp_iso_table", (0, 0.0))[0]
+
+    for (p, s, coils), (_, _, launches) in zip(objs, cases):  # alone
+        ticket = server.submit_simulate_signal(p, s, traj, coils)
+        assert server.wait(ticket, timeout=60) is not None
+        server.release(ticket)
+        assert sub_step_launches() == launches
+    tickets = [server.submit_simulate_signal(p, s, traj, coils) for p, s, coils in objs]  # together
+    for ticket, (p, s, coils) in zip(tickets, objs):
+        assert server.wait(ticket, timeout=60) is not None
+        got, want = server.result(ticket, 0).collect(), ca.simulate_magnetization(p, s).collect()
+        bad = np.isnan(want)
+        assert np.array_equal(np.isnan(got), bad)
+        # FP64 recursions of one form; the positions are summed in FP32 groups of
+        # another size: 3e-7 as for the plain call against the oracle
+        assert rel(got[~bad], want[~bad]) < 3e-7
+    assert sub_step_launches() >= 2
+    for ticket in tickets:
+        server.release(ticket)
+    # the perturbed simulations of a J^H.y request, one after the other
+    p, s, coils = ca.TissueParameters.from_tissue(small), objs[1][1], objs[2][2]
+    y = ca.CompasArray.from_numpy(np.ones((1, nTR, 16), np.complex64))
+    ticket = server.submit_jacobian_hermitian(p, s, traj, coils, y)
+    assert server.wait(ticket, timeout=60) is not None
+    assert sub_step_launches() == 5
+    assert np.all(np.isfinite(server.result(ticket, 1).collect()))
+    server.release(ticket)
+    server.close()
