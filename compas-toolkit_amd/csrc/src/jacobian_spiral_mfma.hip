@@ -44,6 +44,7 @@
 #include "compas/device/mfma_tile.h"
 #include "compas/device/spiral_phasor.h"
 #include "compas/internal.h"
+#include "compas/spiral_layout.h"
 
 namespace compas {
 namespace kernels {
@@ -280,75 +281,42 @@ bool spiral_hermitian_mfma(
     const cfloat* db1, const cfloat* db0, const cfloat* coils, int nc, const cfloat* y, const SpiralTrajectory& traj,
     ContractionPrecision precision, cfloat* JHy) {
     if (precision == ContractionPrecision::FP32) return false;
-    if (nc > 8) return false;  // more coils: the VALU form
+    if (nc > SPIRAL_ADJOINT_COILS) return false;  // the VALU form
     const bool lo = precision == ContractionPrecision::BF16x3 || precision == ContractionPrecision::FP16x3;
     const int nr = traj.nreadouts, ns = traj.samples_per_readout, nv = p.nvoxels;
     // one voxel tile in each of twelve waves, three to a SIMD (at 4 coils x 1120 x
     // 512 over 50176 voxels 5.7 ms; two tiles in each of eight waves spilled, 5.9;
     // sixteen waves 6.3)
-    constexpr int T = 1, W = 12;
-    // four t of the smallest S that holds the samples, eight t of S = 64 for more
-    // than 256, blocks of 512 beyond
-    const int ks = ns <= 32 ? 1 : ns <= 64 ? 2 : ns <= 128 ? 4 : 8;
-    const bool t8 = ns > 256;
-    const int groups = int(dev::div_ceil(nc, t8 ? 4 : 8));
-    const int blocks = groups * int(dev::div_ceil(ns, 8 * ks * (t8 ? 8 : 4)));
-    const size_t words = size_t(ks) * kernels::SHM_TILES * (lo ? 2 : 1) * 64;
-    auto frag = ctx.empty<uint4, 1>({int64_t(nr) * blocks * int64_t(words)});
+    constexpr int T = SPIRAL_ADJOINT_VOXELS / 32, W = SPIRAL_ADJOINT_WAVES;
+    const SpiralAdjointLayout l = spiral_adjoint_layout(nv, nr, ns, nc, lo, simd_count(ctx.device()) / 4);
+    auto frag = ctx.empty<uint4, 1>({l.fragment_bytes(nr) / int64_t(sizeof(uint4))});
     auto voxels = spiral_voxel_table(ctx, p, traj.delta_t);
-    const int vblocks = int(dev::div_ceil(nv, 32 * T * W));
+    auto partial = ctx.empty<cfloat, 1>({l.partial_bytes(nv) / int64_t(sizeof(cfloat))});
     const auto run = [&](auto ks_c, auto t8_c, auto lo_c) {
         constexpr int KS = decltype(ks_c)::value;
         constexpr bool T8 = decltype(t8_c)::value, LO = decltype(lo_c)::value;
         {
             KernelScope scope(ctx, "spiral_y_fragments");
-            kernels::spiral_y_fragments<KS, T8, LO><<<dim3(nr, blocks), 64 * KS, 0, ctx.stream()>>>(
-                y, nc, nr, ns, groups, frag.data());
+            kernels::spiral_y_fragments<KS, T8, LO><<<dim3(nr, l.blocks), 64 * KS, 0, ctx.stream()>>>(
+                y, nc, nr, ns, l.groups, frag.data());
             check_launch("spiral_y_fragments");
         }
-        // readout chunks: the fewest rounds of resident workgroups times a chunk's
-        // readouts (and two readouts' worth of beginning and end).  A chunk is summed
-        // in FP32 and the chunks in FP64, so a chunk is no longer than 192 readouts
-        // (98304 voxels x 1120 readouts in one chunk: 4.9e-7 of a constant sum, in
-        // six 8e-8)
-        static const int resident = [] {
-            int n = 0;
-            COMPAS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &n, kernels::spiral_hermitian_mfma<T, W, KS, T8, LO>, 64 * W, 0));
-            return std::max(1, n);
-        }();
-        const int64_t slots = int64_t(simd_count(ctx.device()) / 4) * resident;
-        int r_chunk = nr;
-        int64_t best = INT64_MAX;
-        const int fewest = int(dev::div_ceil(nr, 192));
-        for (int n = fewest; n <= nr && (n == fewest || int64_t(n) * vblocks <= 8 * slots); n++) {
-            const int size = int(dev::div_ceil(nr, n));
-            const int64_t cost = int64_t(dev::div_ceil(int64_t(dev::div_ceil(nr, size)) * vblocks, slots)) * (size + 2);
-            if (cost < best) {
-                best = cost;
-                r_chunk = size;
-            }
-        }
-        const int chunks = int(dev::div_ceil(nr, r_chunk));
-        auto partial = ctx.empty<cfloat, 1>({int64_t(chunks) * 6 * nv});
-        {
-            KernelScope scope(ctx, "spiral_hermitian_mfma");
-            kernels::spiral_hermitian_mfma<T, W, KS, T8, LO><<<dim3(vblocks, chunks), 64 * W, 0, ctx.stream()>>>(
-                voxels.data(), dev::tissue_view(p), m, d1, d2, db1, db0, coils, nc, frag.data(), blocks, groups,
-                traj.k_start.data(), traj.delta_k.data(), nr, ns, traj.delta_t, r_chunk, partial.data());
-            check_launch("spiral_hermitian_mfma");
-        }
-        spiral_hermitian_reduce_partials(ctx, partial.data(), chunks, nv, JHy);
+        KernelScope scope(ctx, "spiral_hermitian_mfma");
+        kernels::spiral_hermitian_mfma<T, W, KS, T8, LO><<<dim3(l.vblocks, l.chunks), 64 * W, 0, ctx.stream()>>>(
+            voxels.data(), dev::tissue_view(p), m, d1, d2, db1, db0, coils, nc, frag.data(), l.blocks, l.groups,
+            traj.k_start.data(), traj.delta_k.data(), nr, ns, traj.delta_t, l.r_chunk, partial.data());
+        check_launch("spiral_hermitian_mfma");
     };
     const auto with_lo = [&](auto ks_c, auto t8_c) {
         if (lo) run(ks_c, t8_c, std::true_type {});
         else run(ks_c, t8_c, std::false_type {});
     };
-    if (ks == 1) with_lo(std::integral_constant<int, 1> {}, std::false_type {});
-    else if (ks == 2) with_lo(std::integral_constant<int, 2> {}, std::false_type {});
-    else if (ks == 4) with_lo(std::integral_constant<int, 4> {}, std::false_type {});
-    else if (!t8) with_lo(std::integral_constant<int, 8> {}, std::false_type {});
+    if (l.ks == 1) with_lo(std::integral_constant<int, 1> {}, std::false_type {});
+    else if (l.ks == 2) with_lo(std::integral_constant<int, 2> {}, std::false_type {});
+    else if (l.ks == 4) with_lo(std::integral_constant<int, 4> {}, std::false_type {});
+    else if (!l.t8) with_lo(std::integral_constant<int, 8> {}, std::false_type {});
     else with_lo(std::integral_constant<int, 8> {}, std::true_type {});
+    spiral_hermitian_reduce_partials(ctx, partial.data(), l.chunks, nv, JHy);
     return true;
 }
 

@@ -39,6 +39,7 @@
 #include "compas/device/pssfp_common.h"
 #include "compas/device/pssfp_map.h"
 #include "compas/internal.h"
+#include "compas/spiral_layout.h"
 
 namespace compas {
 
@@ -335,7 +336,12 @@ size_t Server::estimate_bytes(const ServeRequest& r) const {
         // derivatives (each computed in place over its perturbed simulation),
         // the decay operand and the partial sums of the contraction
         bytes += nder * echo + 16 * nv * ns + 2 * echo;
-        if (!r.cartesian) bytes += nr * (size_t(128) << 10);  // the residual as operand fragments
+        if (!r.cartesian && nv * nr * ns * nc > 0 && nc <= SPIRAL_ADJOINT_COILS) {
+            // the residual as operand fragments (at most hi + lo) and the partial sums
+            const auto l = spiral_adjoint_layout(
+                int(nv), int(nr), int(ns), int(nc), true, simd_count(base_.device()) / 4);
+            bytes += size_t(l.fragment_bytes(int(nr)) + l.partial_bytes(int(nv)));
+        }
     }
     return bytes;
 }

@@ -307,3 +307,24 @@ def test_pssfp_beyond_the_maps_is_cut_into_items():
     assert np.all(np.isfinite(server.result(ticket, 1).collect()))
     server.release(ticket)
     server.close()
+
+
+def test_memory_budget_counts_the_residual_operand():
+    """A spiral J^H.y of 8 coils x 1000 readouts x 2048 samples lays its residual
+    out in 512 MiB of operand fragments: two do not fit 800 MiB at once."""
+    banner("serving: memory of the spiral residual operand")
+    context()
+    nr, ns, nc = 1000, 2048, 8
+    t = W.make_tissue(W.SplitMix64(9), 8, 20.0, 40.0)
+    p = ca.TissueParameters.from_tissue(t)
+    s = ca.FispSequence.from_sequence(W.make_fisp(nr, 60.0, 5))
+    traj = ca.SpiralTrajectory.from_trajectory(W.make_spiral(nr, ns, 20.0, 8, 5e-6))
+    coils = ca.CompasArray.from_numpy(np.ones((nc, 64), np.complex64))
+    y = ca.CompasArray.from_numpy(np.ones((nc, nr, ns), np.complex64))
+    server = ca.Server(slots=2, memory_budget=800 << 20)
+    tickets = [server.submit_jacobian_hermitian(p, s, traj, coils, y) for _ in range(2)]
+    (_, _, done), (_, start, _) = [server.wait(k, timeout=60) for k in tickets]
+    for k in tickets:
+        server.release(k)
+    server.close()
+    assert start >= done
