@@ -49,7 +49,11 @@ constexpr int MAP_PHASE = MAP_NODES;  // first of the four phase entries
 struct PssfpMapArgs {
     PssfpArgs a;
     const double* train;  // [1 + nTR][MAP_ROW]
-    cfloat* partial;      // partial planes of the slice-position groups after the first
+    // several slice-position groups: an FP64 plane of each, so that the sum is
+    // rounded once (FP32 planes after the first: 3.0e-8 instead of 2.5e-8 on the
+    // tangents of 35 positions in three groups).  Or, in the same memory, the FP32
+    // planes of the sub-step form's groups after the first
+    cfloat* partial;
     int nv_block;         // voxels of a workgroup
     int nz_group;         // slice positions of a group (nv_block nz_group <= 256)
     int vblocks, groups;  // ceil(nv / nv_block), ceil(nz / nz_group)

@@ -142,15 +142,12 @@ bool spiral_hermitian_mfma(
 // JHy[p][v] = sum over `chunks` partial [6][nv] planes (FP64)
 void spiral_hermitian_reduce_partials(const CompasContext& ctx, const cfloat* partial, int chunks, int nv, cfloat* JHy);
 
-// device bytes of partial echoes one pSSFP simulation of this size allocates
-int64_t pssfp_scratch_bytes(const CompasContext& ctx, int nz, int nv, int nTR);
-
 // echos[i] += sum over count partial planes of n elements (plane j at
 // partial + j * stride), in FP64, in order; with the table of a train, only if
-// the maps served it (`mapped`) or only if they did not
+// the maps did not serve it
 void pssfp_sum_groups(
     const CompasContext& ctx, cfloat* echos, const cfloat* partial, int count, int64_t n, int64_t stride,
-    const double* train = nullptr, bool mapped = false);
+    const double* train = nullptr);
 
 // Work-table launches of the request server: workgroup b runs items[b].
 //   FISP: item (job, voxel block of 64), every job with max_state == spl,
@@ -167,11 +164,13 @@ void launch_pssfp_table(
 // The simulation by one affine map per isochromat and TR (pssfp_map.hip):
 // whether it pays for a train; the doubles of the train's table; the launch
 // arguments, with the table's kernel enqueued (`zpl`: slice positions per lane
-// of the sub-step form, should the train be beyond the maps); the partial
-// planes that either form needs; the workgroups of the maps, launched for one
-// simulation (jobs == nullptr) or as items (job, unit) of a work table; the
-// sub-step form, which does nothing where the maps served; and what follows
-// the maps: that form and the sum of the partial planes.
+// of the sub-step form, should the train be beyond the maps); the echo planes
+// (of complex FP32 size) that their partial sums take; the workgroups of the
+// maps, launched for one simulation (jobs == nullptr) or as items (job, unit) of
+// a work table; the sum of the partial planes (out[i] = sum_j partial[j stride +
+// i], FP64), which does nothing where the maps did not serve or there is one
+// group; the sub-step form, which does nothing where they did; and what follows
+// the maps: that sum, that form and its sum.
 bool pssfp_map_pays(int nTR, int nRF);
 int64_t pssfp_map_train_size(int nTR);
 constexpr int pssfp_map_served_entry = 1;  // of the table: not 0 if the maps serve the train
@@ -181,6 +180,9 @@ int64_t pssfp_map_units(const kernels::PssfpMapArgs& p);
 void launch_pssfp_map(
     const CompasContext& ctx, const kernels::PssfpMapArgs& single, const kernels::PssfpMapArgs* jobs,
     const int2* items, int64_t n);
+void pssfp_map_sum(
+    const CompasContext& ctx, cfloat* out, const cfloat* partial, int groups, int64_t n, int64_t stride,
+    const double* train);
 void launch_pssfp_unmapped(const CompasContext& ctx, const kernels::PssfpMapArgs& p);
 void pssfp_map_finish(const CompasContext& ctx, const kernels::PssfpMapArgs& p);
 

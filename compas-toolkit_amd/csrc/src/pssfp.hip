@@ -227,12 +227,12 @@ __global__ void __launch_bounds__(64) pssfp_iso_table(const PssfpTableJob* __res
 }
 
 // echos[i] += sum_j partial[j][i], accumulated in FP64 in slot order
-// (train: nullptr, or the table of a train: nothing is done unless the maps
-// served it, or did not, as `mapped` says)
+// (train: nullptr, or the table of a train: nothing is done where the maps served
+// it)
 __global__ void pssfp_sum_groups_kernel(
     cfloat* __restrict__ echos, const cfloat* __restrict__ partial, int count, int64_t n, int64_t stride,
-    const double* train, bool mapped) {
-    if (train != nullptr && (train[1] != 0.0) != mapped) return;
+    const double* train) {
+    if (train != nullptr && train[1] != 0.0) return;
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
         const cfloat e = echos[i];
         double re = e.re, im = e.im;
@@ -249,11 +249,11 @@ __global__ void pssfp_sum_groups_kernel(
 
 void pssfp_sum_groups(
     const CompasContext& ctx, cfloat* echos, const cfloat* partial, int count, int64_t n, int64_t stride,
-    const double* train, bool mapped) {
+    const double* train) {
     if (count <= 0 || n == 0) return;
     KernelScope ks(ctx, "pssfp_sum_groups");
     const int64_t blocks = std::min<int64_t>(dev::div_ceil(n, int64_t(256)), 8192);
-    kernels::pssfp_sum_groups_kernel<<<unsigned(blocks), 256, 0, ctx.stream()>>>(echos, partial, count, n, stride, train, mapped);
+    kernels::pssfp_sum_groups_kernel<<<unsigned(blocks), 256, 0, ctx.stream()>>>(echos, partial, count, n, stride, train);
     check_launch("pssfp_sum_groups");
 }
 
@@ -376,11 +376,6 @@ static int partial_slots(const PssfpLayout& L) {
     return L.groups > L.per_launch ? L.per_launch : L.groups - 1;
 }
 
-int64_t pssfp_scratch_bytes(const CompasContext& ctx, int nz, int nv, int nTR) {
-    if (nz <= 0 || nv <= 0 || nTR <= 0) return 0;
-    return int64_t(partial_slots(primal_layout(ctx, nz, nv, nTR))) * nTR * nv * int64_t(sizeof(cfloat));
-}
-
 Array<cfloat, 2> simulate_magnetization(
     const CompasContext& ctx,
     TissueParameters parameters,
@@ -421,7 +416,8 @@ Array<cfloat, 2> simulate_magnetization(
         kernels::PssfpMapArgs p {};
         pssfp_map_setup(ctx, p, a, train.data(), L.zpl);
         Array<cfloat, 2> part;
-        if (const int planes = pssfp_map_partial_planes(p)) part = ctx.empty<cfloat, 2>({planes, plane});
+        const int planes = std::max(pssfp_map_partial_planes(p), p.direct_groups - 1);
+        if (planes > 0) part = ctx.empty<cfloat, 2>({planes, plane});
         p.partial = part.data();
         launch_pssfp_map(ctx, p, nullptr, nullptr, pssfp_map_units(p));
         pssfp_map_finish(ctx, p);

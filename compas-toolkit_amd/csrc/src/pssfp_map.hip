@@ -18,8 +18,8 @@
 //     its transverse magnetisation into LDS, and every MAP_CHUNK TRs the
 //     workgroup adds up the previous chunk (FP64, in order of position) while
 //     it computes the next; two LDS buffers, one barrier per chunk.  No partial
-//     echoes go through HBM unless there are more than about a hundred slice
-//     positions.
+//     echoes go through HBM unless there are more than about eighty slice
+//     positions; then each group has an FP64 plane.
 //   * Neighbouring voxel blocks run on one XCD, so that the 8 nv_block bytes a
 //     workgroup writes per TR meet their neighbours' in that XCD's L2.
 //   * What bounds it: FP64 issue.  At 50176 voxels x 1120 TRs x 35 positions the
@@ -131,11 +131,10 @@ __device__ __forceinline__ void pulse(const IsoConst& k, const double2* grf, int
 }
 
 // The echoes of nv_block voxels x nz_group slice positions; `block` and `group`
-// name them, out is the group's echo plane [nTR][nv].
+// name them.
 template<bool PHASED>
 __device__ __forceinline__ void pssfp_map_block(
-    const PssfpMapArgs& p, int block, int group, cfloat* __restrict__ out, const double2* grf,
-    double2 (*sums)[MAP_CHUNK][256]) {
+    const PssfpMapArgs& p, int block, int group, const double2* grf, double2 (*sums)[MAP_CHUNK][256]) {
     const PssfpArgs& a = p.a;
     const int tid = threadIdx.x;
     const int nv = a.tissue.nvoxels;
@@ -247,7 +246,12 @@ __device__ __forceinline__ void pssfp_map_block(
                     y = r[0] * y - r[1] * x;
                     x = xr;
                 }
-                out[size_t(n) * nv + v0 + w] = {float(x), float(y)};
+                const size_t at = size_t(n) * nv + v0 + w;
+                if (p.groups == 1) {
+                    a.echos[at] = {float(x), float(y)};
+                } else {
+                    reinterpret_cast<double2*>(p.partial)[size_t(group) * a.nTR * nv + at] = make_double2(x, y);
+                }
             }
         }
     };
@@ -309,29 +313,27 @@ __global__ void __launch_bounds__(256, 2) pssfp_map(
     for (int i = threadIdx.x; i < p.a.nRF; i += 256) grf[i] = make_double2(double(p.a.gamma_dt_RF[i].re), double(p.a.gamma_dt_RF[i].im));
     __syncthreads();
     const int group = unit / p.vblocks;
-    cfloat* out = group == 0 ? p.a.echos : p.partial + size_t(group - 1) * size_t(p.a.nTR) * size_t(p.a.tissue.nvoxels);
     if (p.train[2] != 0.0) {
-        pssfp_map_block<true>(p, unit % p.vblocks, group, out, grf, sums);
+        pssfp_map_block<true>(p, unit % p.vblocks, group, grf, sums);
     } else {
-        pssfp_map_block<false>(p, unit % p.vblocks, group, out, grf, sums);
+        pssfp_map_block<false>(p, unit % p.vblocks, group, grf, sums);
     }
 }
 
-// echos[i] += sum_j partial[j][i] over the groups of the form that ran, in
-// FP64 and in order
-__global__ void pssfp_map_sum(cfloat* __restrict__ echos, const cfloat* __restrict__ partial, const double* train,
-                              int map_groups, int direct_groups, int64_t n) {
-    const int count = (train[1] != 0.0 ? map_groups : direct_groups) - 1;
-    if (count <= 0) return;
+// out[i] = sum over the groups' planes (plane j at partial + j stride), in
+// order; nothing where the maps did not serve the train
+__global__ void pssfp_map_sum(
+    cfloat* __restrict__ out, const double2* __restrict__ partial, int groups, int64_t n, int64_t stride,
+    const double* train) {
+    if (train[1] == 0.0) return;
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
-        const cfloat e = echos[i];
-        double re = e.re, im = e.im;
-        for (int j = 0; j < count; j++) {
-            const cfloat q = partial[size_t(j) * size_t(n) + size_t(i)];
-            re += q.re;
-            im += q.im;
+        double re = 0.0, im = 0.0;
+        for (int j = 0; j < groups; j++) {
+            const double2 q = partial[size_t(j) * size_t(stride) + size_t(i)];
+            re += q.x;
+            im += q.y;
         }
-        echos[i] = {float(re), float(im)};
+        out[i] = {float(re), float(im)};
     }
 }
 
@@ -377,7 +379,7 @@ void pssfp_map_setup(const CompasContext& ctx, kernels::PssfpMapArgs& p, const k
 }
 
 int pssfp_map_partial_planes(const kernels::PssfpMapArgs& p) {
-    return std::max(p.groups, p.direct_groups) - 1;
+    return p.groups > 1 ? 2 * p.groups : 0;
 }
 
 int64_t pssfp_map_units(const kernels::PssfpMapArgs& p) {
@@ -393,15 +395,22 @@ void launch_pssfp_map(
     check_launch("pssfp_map");
 }
 
-void pssfp_map_finish(const CompasContext& ctx, const kernels::PssfpMapArgs& p) {
-    launch_pssfp_unmapped(ctx, p);
-    if (pssfp_map_partial_planes(p) <= 0) return;
-    const int64_t n = int64_t(p.a.nTR) * p.a.tissue.nvoxels;
-    KernelScope ks(ctx, "pssfp_sum_groups");
+void pssfp_map_sum(
+    const CompasContext& ctx, cfloat* out, const cfloat* partial, int groups, int64_t n, int64_t stride,
+    const double* train) {
+    if (groups <= 1 || n == 0) return;
+    KernelScope ks(ctx, "pssfp_map_sum");
     const int64_t blocks = std::min<int64_t>(dev::div_ceil(n, int64_t(256)), 8192);
     kernels::pssfp_map_sum<<<unsigned(blocks), 256, 0, ctx.stream()>>>(
-        p.a.echos, p.partial, p.train, p.groups, p.direct_groups, n);
+        out, reinterpret_cast<const double2*>(partial), groups, n, stride, train);
     check_launch("pssfp_map_sum");
+}
+
+void pssfp_map_finish(const CompasContext& ctx, const kernels::PssfpMapArgs& p) {
+    const int64_t n = int64_t(p.a.nTR) * p.a.tissue.nvoxels;
+    pssfp_map_sum(ctx, p.a.echos, p.partial, p.groups, n, n, p.train);
+    launch_pssfp_unmapped(ctx, p);
+    pssfp_sum_groups(ctx, p.a.echos, p.partial, p.direct_groups - 1, n, n, p.train);
 }
 
 }  // namespace compas

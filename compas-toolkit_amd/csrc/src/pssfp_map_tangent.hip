@@ -86,8 +86,8 @@ __device__ inline Mat3 rotation_derivative(
 }
 
 struct MapTangentArgs {
-    PssfpMapArgs p;  // partial: planes of the groups after the first, NP each
-    cfloat* out[3];  // output planes of group 0, in the order of TangentSet
+    PssfpMapArgs p;  // partial: NP planes of each group
+    cfloat* out[3];  // output planes, in the order of TangentSet
     double* nodes;   // [1 + NT maps][MAP_NODES][MAP_ENTRIES][isos], then [3 + 3 NT][isos]
     int v0, nv;      // voxels of this launch
 };
@@ -385,9 +385,13 @@ __device__ __forceinline__ void pssfp_map_tangents_block(const MapTangentArgs& t
                     y = r[0] * y - r[1] * x;
                     x = xr;
                 }
-                cfloat* o = k == 0 ? t.out[0] : k == 1 ? t.out[1] : t.out[2];
-                if (group > 0) o = t.p.partial + (size_t(group - 1) * NP + k) * plane;
-                o[size_t(n) * nv_all + t.v0 + v0 + vox] = {float(x), float(y)};
+                const size_t at = size_t(n) * nv_all + t.v0 + v0 + vox;
+                if (t.p.groups == 1) {
+                    cfloat* o = k == 0 ? t.out[0] : k == 1 ? t.out[1] : t.out[2];
+                    o[at] = {float(x), float(y)};
+                } else {
+                    reinterpret_cast<double2*>(t.p.partial)[(size_t(group) * NP + k) * plane + at] = make_double2(x, y);
+                }
             }
         }
     };
@@ -495,7 +499,7 @@ void run_pass(const CompasContext& ctx, const PssfpArgs& a, const double* train,
     t.p.groups = w.groups;
     const int64_t plane = int64_t(a.nTR) * a.tissue.nvoxels;
     Array<cfloat, 2> part;
-    if (t.p.groups > 1) part = ctx.empty<cfloat, 2>({int64_t(t.p.groups - 1) * NP, plane});
+    if (t.p.groups > 1) part = ctx.empty<cfloat, 2>({int64_t(pssfp_map_partial_planes(t.p)) * NP, plane});
     t.p.partial = part.data();
     // node values of at most about 1 GiB of isochromats at a time
     const int64_t per_iso = int64_t((1 + NT) * MAP_NODES * MAP_ENTRIES + 3 + 3 * NT) * 8;
@@ -516,7 +520,7 @@ void run_pass(const CompasContext& ctx, const PssfpArgs& a, const double* train,
         check_launch("pssfp_map_tangents");
     }
     for (int k = 0; k < NP; k++)
-        pssfp_sum_groups(ctx, planes[k], part.data() + k * plane, t.p.groups - 1, plane, NP * plane, train, true);
+        pssfp_map_sum(ctx, planes[k], part.data() + 2 * k * plane, t.p.groups, plane, NP * plane, train);
 }
 
 }  // namespace

@@ -615,7 +615,7 @@ void run_pass(const CompasContext& ctx, int mask, const kernels::PssfpArgs& a, c
         }
         const int summed = g0 == 0 ? count - 1 : count;
         for (int k = 0; k < np; k++)
-            pssfp_sum_groups(ctx, planes[k], part.data() + k * plane, summed, plane, np * plane, train, false);
+            pssfp_sum_groups(ctx, planes[k], part.data() + k * plane, summed, plane, np * plane, train);
     }
     if (train != nullptr) launch_pssfp_map_tangents(ctx, mask, a, train, planes);
 }

@@ -182,7 +182,8 @@ void make_items(const CompasContext& sim, Server::SimJob& j, bool maps) {
         j.item_cost =
             double(a.nTR + 1) * std::max(a.nRF, 1) * (j.bucket * 50.0 + 12.0) + double(a.nTR) * j.bucket * 40.0;
     }
-    if (j.groups > 1) j.partial = sim.empty<cfloat, 2>({j.groups - 1, int64_t(a.nTR) * a.tissue.nvoxels});
+    const int planes = maps ? pssfp_map_partial_planes(j.map) : j.groups - 1;
+    if (planes > 0) j.partial = sim.empty<cfloat, 2>({planes, int64_t(a.nTR) * a.tissue.nvoxels});
     j.map.partial = j.pss.partial = j.partial.data();
 }
 
@@ -512,7 +513,10 @@ void Server::complete_jobs() {
             for (int st = 1; st < kSimStreams; st++) {
                 if (j.last[st]) COMPAS_HIP_CHECK(hipStreamWaitEvent(sim.stream(), j.last[st]->ev, 0));
             }
-            if (j.pssfp && j.groups > 1) {
+            if (j.maps) {
+                pssfp_map_sum(sim, j.echos.data(), j.partial.data(), j.groups, j.echos.numel(), j.echos.numel(),
+                              j.train.data());
+            } else if (j.pssfp && j.groups > 1) {
                 const int64_t plane = j.echos.numel();
                 pssfp_sum_groups(sim, j.echos.data(), j.partial.data(), j.groups - 1, plane, plane);
             }

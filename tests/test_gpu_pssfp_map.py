@@ -113,3 +113,23 @@ def test_many_slice_positions(oracle):
     assert np.array_equal(server.result(ticket, 0).collect(), got)
     server.release(ticket)
     server.close()
+
+
+@pytest.mark.parametrize("nz,tangents", [(35, True), (200, False)], ids=["tangents", "simulation"])
+def test_sums_of_groups_are_rounded_once(oracle, nz, tangents):
+    """Slice positions in several groups: the sums are FP64 up to the echo, so the
+    error is that of rounding the oracle's echoes to FP32.  FP32 planes of two or
+    three groups would leave 1.15 times that or more; 1.03."""
+    banner(f"pssfp map, rounding of {nz} positions")
+    context()
+    t = W.make_tissue(W.SplitMix64(77), 20, 20.0, 40.0)
+    seq = train(80, 60.0, nz, 25, 0.0)
+    p, s = ca.TissueParameters.from_tissue(t), ca.pSSFPSequence.from_sequence(seq)
+    if tangents:
+        got = ca.simulate_magnetization_tangents((ca.T1, ca.T2), p, s, echos=True)[0].collect()
+    else:
+        got = ca.simulate_magnetization(p, s).collect()
+    want = oracle.pssfp(t, seq, "f64")
+    once = rel(want.astype(np.complex64), want)
+    print("error", rel(got, want), "of one rounding", once)
+    assert rel(got, want) < 1.03 * once
