@@ -1,8 +1,7 @@
 """FISP trains of real pulses (fisp_real.h) against the FP64 oracle, where the
-layout or the form changes: one lane per voxel and several (the top state in
-each of the last places of its lane), the options that leave the plain loop,
-flip angles of either sign and beyond the polynomial's range, and trains that
-are real but for one pulse (the complex form).
+layout or the form changes: one lane per voxel and several, the options that
+leave the plain loop, flip angles of either sign and beyond the polynomial's
+range, and trains that are real but for one pulse (the complex form).
 
 Tolerance: the recursion is the one the complex form runs, in FP32, with fewer
 roundings; 1e-5 (echoes) and 1e-4 (tangents) relative to FP64 are the bounds of
@@ -31,7 +30,8 @@ def case(nv, nTR, N, deg=60.0, b0=40.0):
     return t, seq
 
 
-# (voxels, states): few voxels take eight lanes, 30000 four or two, 80000 one
+# (voxels, states) by the layout rule for 1024 SIMDs: 33 voxels take eight lanes
+# from seven states on, 30000 one or two, 80000 one, and four for 40 states
 LAYOUTS = [(33, 1), (33, 2), (33, 7), (33, 8), (33, 9), (33, 25), (33, 33), (33, 63), (33, 128), (30000, 3),
            (30000, 25), (30000, 32), (80000, 13), (80000, 32), (80000, 40)]
 
@@ -41,6 +41,19 @@ def test_layouts(oracle, nv, N):
     banner(f"fisp real layouts {nv} voxels {N} states")
     context()
     t, seq = case(nv, 30, N)
+    got = ca.simulate_magnetization(ca.TissueParameters.from_tissue(t), ca.FispSequence.from_sequence(seq)).collect()
+    assert rel(got, oracle.fisp(t, seq, "f64")) < MAG_TOL
+
+
+# every lane count with the top state in each of the last places of its lane
+@pytest.mark.parametrize("lanes,N", [(1, 1), (1, 2), (1, 32), (2, 2), (2, 3), (2, 31), (2, 32), (4, 4), (4, 5), (4, 6), (4, 7),
+                                     (4, 13), (4, 14), (4, 15), (4, 16), (4, 61), (4, 62), (4, 63), (4, 64), (8, 9), (8, 23),
+                                     (8, 121), (8, 125), (8, 128)])
+def test_lanes(oracle, monkeypatch, lanes, N):
+    banner(f"fisp real, {N} states in {lanes} lanes")
+    monkeypatch.setenv("COMPAS_FISP_LPV", str(lanes))
+    context()
+    t, seq = case(9, 33, N)
     got = ca.simulate_magnetization(ca.TissueParameters.from_tissue(t), ca.FispSequence.from_sequence(seq)).collect()
     assert rel(got, oracle.fisp(t, seq, "f64")) < MAG_TOL
 
