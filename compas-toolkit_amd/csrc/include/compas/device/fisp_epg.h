@@ -163,16 +163,9 @@ __device__ __forceinline__ void fisp_epg_voxel_form(const FispArgs& a, int voxel
                     const float xr = fmaf(h00, S.re, fmaf(h01, D.im, M02 * z.re));
                     const float yr = fmaf(h10, S.re, fmaf(h11, D.im, M12 * z.re));
                     const float zr = fmaf(h20, S.re, fmaf(h21, D.im, M22 * z.re));
-                    float xi, yi, zi;
-                    if (false) {
-                        xi = M02 * z.im;
-                        yi = M12 * z.im;
-                        zi = M22 * z.im;
-                    } else {
-                        xi = fmaf(h00, S.im, fmaf(-h01, D.re, M02 * z.im));
-                        yi = fmaf(h10, S.im, fmaf(-h11, D.re, M12 * z.im));
-                        zi = fmaf(h20, S.im, fmaf(-h21, D.re, M22 * z.im));
-                    }
+                    const float xi = fmaf(h00, S.im, fmaf(-h01, D.re, M02 * z.im));
+                    const float yi = fmaf(h10, S.im, fmaf(-h11, D.re, M12 * z.im));
+                    const float zi = fmaf(h20, S.im, fmaf(-h21, D.re, M22 * z.im));
                     const cfloat pn = {xr - yi, xi + yr}, qn = {xr + yi, xi - yr};
                     if (i == 0) pn0 = pn;
                     if (i + 1 < SPL) {

@@ -39,6 +39,9 @@ constexpr double MAP_SQRT_X[MAP_NODES] = {0.9951847266721969, 0.0980171403295607
                                           0.8819212643483549, 0.4713967368259978, 0.9569403357322088,
                                           0.29028467725446233, 0.773010453362737};
 
+// Entries of a map: the first six even in theta, the last six odd
+enum MapEntry : int { MXX, MXY, MYX, MYY, MZZ, MCZ, MXZ, MYZ, MZX, MZY, MCX, MCY, MAP_ENTRIES };
+
 // Row n of a train's table: theta_n (in units of the largest amplitude), x_n -
 // MAP_X[j] for j < MAP_NODES - 1, then cos and sin of phi_n - phi_{n-1}, and of
 // phi_n.  Row -1 (the header, first in memory) holds the largest amplitude,

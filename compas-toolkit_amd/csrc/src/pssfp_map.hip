@@ -111,9 +111,6 @@ __global__ void __launch_bounds__(1024) pssfp_map_train(PssfpArgs a, double* tra
     }
 }
 
-// Entries of a map: the first six even in theta, the last six odd
-enum MapEntry : int { MXX, MXY, MYX, MYY, MZZ, MCZ, MXZ, MYZ, MZX, MZY, MCX, MCY, MAP_ENTRIES };
-
 // One RF pulse of amplitude rf: nv vectors through the sub-steps, the last of
 // them with regrowth (the others are the columns of the linear part)
 template<int NV>

@@ -38,9 +38,6 @@ namespace kernels {
 
 constexpr int MAPT_CHUNK = 8;  // TRs summed over slice positions at a time
 
-// Entries of a map, the first six even in theta; as in pssfp_map.hip
-enum MapEntry : int { MXX, MXY, MYX, MYY, MZZ, MCZ, MXZ, MYZ, MZX, MZY, MCX, MCY, MAP_ENTRIES };
-
 // v of the lane that the quad permutation names
 template<int CONTROL>
 __device__ __forceinline__ double quad(double v) {
