@@ -17,6 +17,18 @@ struct alignas(16) SpiralVoxel {
     float pad[2];
 };
 
+// Written beside a kernel that runs before the products anyway: a launch of its
+// own made the smallest calls slower than the products gained
+__device__ inline SpiralVoxel spiral_voxel(const dev::TissueView& t, float dt, int v) {
+    SpiralVoxel o {};
+    o.turns = double(dt) * double(t.B0(v));
+    o.x = t.x(v);
+    o.y = t.y(v);
+    o.T2 = t.T2(v);
+    o.decay = float(-1.4426950408889634 * double(dt) / double(o.T2));  // log2(e)
+    return o;
+}
+
 // Turns per sample of a voxel; dkx, dky: delta_k / 2 pi
 __device__ __forceinline__ double spiral_turns(const SpiralVoxel& v, double dkx, double dky) {
     return fma(dkx, double(v.x), fma(dky, double(v.y), v.turns));
@@ -37,8 +49,4 @@ __device__ __forceinline__ cfloat spiral_phasor(float log2_mag, double turns) {
 }
 
 }  // namespace kernels
-
-// The voxels' constants, on the context's stream (signal_spiral_mfma.hip)
-Array<kernels::SpiralVoxel, 1> spiral_voxel_table(const CompasContext& ctx, const TissueParameters& p, float dt);
-
 }  // namespace compas

@@ -14,6 +14,7 @@ struct FispPlanes;
 struct PssfpArgs;
 struct PssfpTableJob;
 struct PssfpMapArgs;
+struct SpiralVoxel;
 }  // namespace kernels
 
 // dst[i] += src[i] for i < n (complex)
@@ -93,16 +94,19 @@ bool jacobian_hermitian_mfma(
 // Spiral sum out[c][r][s] = sum_v C[c][v] (A[r][v] + (s - ns/2) Ab[r][v]) E_rv^s
 // with the per-readout sample exponent of the spiral trajectory (Ab may be
 // nullptr).  A and Ab already carry the readout factor (rewind, prephaser).
+// voxels: the voxels' constants (spiral_voxel), for the sums on MFMA only.
 void spiral_sum(
-    const CompasContext& ctx, const TissueParameters& p, const cfloat* A, const cfloat* Ab, const cfloat* coils,
-    int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out);
+    const CompasContext& ctx, const TissueParameters& p, const kernels::SpiralVoxel* voxels, const cfloat* A,
+    const cfloat* Ab, const cfloat* coils, int nc, const SpiralTrajectory& t, ContractionPrecision precision,
+    cfloat* out);
 
-// The same sums with the voxel contraction on MFMA (BF16 hi + lo, or hi only);
-// false when the precision is FP32 or there are more than eight coils with one
-// amplitude or four with two: the caller runs the VALU form.
-bool spiral_sum_mfma(
-    const CompasContext& ctx, const TissueParameters& p, const cfloat* A, const cfloat* Ab, const cfloat* coils,
-    int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out);
+// The same sums with the voxel contraction on MFMA (BF16 hi + lo, or hi only),
+// and whether they serve: not in FP32, nor for more than eight coils with one
+// amplitude or four with two (the VALU form).
+bool spiral_sum_on_mfma(int nc, bool two, ContractionPrecision precision);
+void spiral_sum_mfma(
+    const CompasContext& ctx, const kernels::SpiralVoxel* voxels, int nv, const cfloat* A, const cfloat* Ab,
+    const cfloat* coils, int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out);
 
 // Per (slice, TR) RF table of the FISP kernels (FispArgs::table).
 Array<float4, 1> fisp_rf_table(const CompasContext& ctx, const FISPSequence& seq);

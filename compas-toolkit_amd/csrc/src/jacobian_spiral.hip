@@ -25,6 +25,7 @@
 // the spiral sum, jacobian_spiral_mfma.hip for J^H.y).
 
 #include "compas/device/common.h"
+#include "compas/device/spiral_phasor.h"
 #include "compas/internal.h"
 
 namespace compas {
@@ -38,16 +39,18 @@ __device__ inline cfloat spiral_readout_factor(const dev::TissueView& t, int v, 
     return dev::polar_f(expf(float(half) * R2), dev::reduce_phase(phi));
 }
 
-// J.v amplitudes times the readout factor: Aa = a Phi0, Ab = b Phi0 ([nr][nv])
+// J.v amplitudes times the readout factor: Aa = a Phi0, Ab = b Phi0 ([nr][nv]);
+// and the voxels' constants for the sums on MFMA, unless nullptr
 __global__ void spiral_jv_amplitudes(
     dev::TissueView t, const cfloat* __restrict__ m, const cfloat* __restrict__ dT1,
     const cfloat* __restrict__ dT2, const cfloat* __restrict__ dB1, const cfloat* __restrict__ dB0,
     const cfloat* __restrict__ vec, const cfloat* __restrict__ k_start, int nr, int ns, float dt,
-    cfloat* __restrict__ Aa, cfloat* __restrict__ Ab) {
+    cfloat* __restrict__ Aa, cfloat* __restrict__ Ab, SpiralVoxel* __restrict__ voxels) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     const int r = blockIdx.y;
     const int nv = t.nvoxels;
     if (v >= nv) return;
+    if (voxels != nullptr && r == 0) voxels[v] = spiral_voxel(t, dt, v);
     const size_t i = size_t(r) * nv + v;
     const cfloat rho = t.rho(v), me = m[i];
     const float T1 = t.T1(v), T2 = t.T2(v), R2 = 1.0f / T2;
@@ -70,7 +73,7 @@ constexpr int JHS_THREADS = 256;  // voxels per workgroup (one per lane)
 constexpr int JHS_ANCHOR = 32;  // samples between FP64-anchored evaluations of Phi
 constexpr int JHS_BLOCK = 8;  // samples per unrolled block (y of the block loaded up front)
 
-struct SpiralVoxel {
+struct SpiralVoxelDirect {
     float R2, decay, T1, T2;
     double B0, x, y, half;
     cfloat rho;
@@ -85,7 +88,7 @@ struct SpiralVoxel {
 // before the block's arithmetic.
 template<int CG>
 __device__ inline void spiral_hermitian_coils(
-    const SpiralVoxel& sv, int vv, int nv, const cfloat* __restrict__ m, const cfloat* __restrict__ dT1,
+    const SpiralVoxelDirect& sv, int vv, int nv, const cfloat* __restrict__ m, const cfloat* __restrict__ dT1,
     const cfloat* __restrict__ dT2, const cfloat* __restrict__ dB1, const cfloat* __restrict__ dB0,
     const cfloat* __restrict__ coils, int cg, const cfloat* __restrict__ y, const cfloat* __restrict__ k_start,
     const cfloat* __restrict__ delta_k, int nr, int ns, float dt, int r0, int r1, cfloat (&out)[6]) {
@@ -184,7 +187,7 @@ __global__ void __launch_bounds__(JHS_THREADS) spiral_hermitian(
     const bool ok = v < nv;
     const int vv = ok ? v : 0;  // out-of-range lanes compute on voxel 0 and store nothing
 
-    SpiralVoxel sv;
+    SpiralVoxelDirect sv;
     sv.T1 = t.T1(vv);
     sv.T2 = t.T2(vv);
     sv.R2 = 1.0f / sv.T2;
@@ -290,15 +293,17 @@ Array<cfloat, 3> compute_jacobian(
     }
     auto Aa = ctx.empty<cfloat, 2>({nr, nv});
     auto Ab = ctx.empty<cfloat, 2>({nr, nv});
+    Array<kernels::SpiralVoxel, 1> voxels;
+    if (spiral_sum_on_mfma(nc, true, precision)) voxels = ctx.empty<kernels::SpiralVoxel, 1>({nv});
     {
         KernelScope ks(ctx, "spiral_jv_amplitudes");
         dim3 grid(dev::div_ceil(nv, 256), nr);
         kernels::spiral_jv_amplitudes<<<grid, 256, 0, ctx.stream()>>>(
             dev::tissue_view(p), echos.data(), dT1.data(), dT2.data(), dB1.data(), dB0.data(), vector.data(),
-            traj.k_start.data(), nr, ns, traj.delta_t, Aa.data(), Ab.data());
+            traj.k_start.data(), nr, ns, traj.delta_t, Aa.data(), Ab.data(), voxels.data());
         check_launch("spiral_jv_amplitudes");
     }
-    spiral_sum(ctx, p, Aa.data(), Ab.data(), coils.data(), nc, traj, precision, Jv.data());
+    spiral_sum(ctx, p, voxels.data(), Aa.data(), Ab.data(), coils.data(), nc, traj, precision, Jv.data());
     return Jv;
 }
 

@@ -62,14 +62,21 @@ __device__ __forceinline__ void shm_row(int row, int& c, int& t) {
 }
 
 // A fragments frag[readout][block][K step][tile][hi, lo][lane], block = sample
-// block x coil group; grid (nr, blocks), block 64 KS.
+// block x coil group; grid (nr + ceil(nv / (64 KS)), blocks), block 64 KS.  The
+// workgroups after the first nr of a row write the voxels' constants.
 template<int KS, bool T8, bool LO>
 __global__ void __launch_bounds__(64 * KS) spiral_y_fragments(
-    const cfloat* __restrict__ y, int nc, int nr, int ns, int groups, uint4* __restrict__ frag) {
+    const cfloat* __restrict__ y, int nc, int nr, int ns, int groups, uint4* __restrict__ frag,
+    dev::TissueView tissue, float dt, SpiralVoxel* __restrict__ voxels) {
     constexpr int P = LO ? mfma::P_BF16X3 : mfma::P_BF16X1;
     constexpr int S = 8 * KS, T = T8 ? 8 : 4, COILS = T8 ? 4 : 8, PARTS = LO ? 2 : 1;
     const int lane = threadIdx.x & 63, ks = threadIdx.x >> 6;
     const int r = blockIdx.x, block = blockIdx.y;
+    if (r >= nr) {
+        const int v = (r - nr) * (64 * KS) + int(threadIdx.x);
+        if (block == 0 && v < tissue.nvoxels) voxels[v] = spiral_voxel(tissue, dt, v);
+        return;
+    }
     int c, t;
     shm_row<T8>(lane & 31, c, t);
     c += COILS * (block % groups);
@@ -290,15 +297,16 @@ bool spiral_hermitian_mfma(
     constexpr int T = SPIRAL_ADJOINT_VOXELS / 32, W = SPIRAL_ADJOINT_WAVES;
     const SpiralAdjointLayout l = spiral_adjoint_layout(nv, nr, ns, nc, lo, simd_count(ctx.device()) / 4);
     auto frag = ctx.empty<uint4, 1>({l.fragment_bytes(nr) / int64_t(sizeof(uint4))});
-    auto voxels = spiral_voxel_table(ctx, p, traj.delta_t);
+    auto voxels = ctx.empty<kernels::SpiralVoxel, 1>({nv});
     auto partial = ctx.empty<cfloat, 1>({l.partial_bytes(nv) / int64_t(sizeof(cfloat))});
     const auto run = [&](auto ks_c, auto t8_c, auto lo_c) {
         constexpr int KS = decltype(ks_c)::value;
         constexpr bool T8 = decltype(t8_c)::value, LO = decltype(lo_c)::value;
         {
             KernelScope scope(ctx, "spiral_y_fragments");
-            kernels::spiral_y_fragments<KS, T8, LO><<<dim3(nr, l.blocks), 64 * KS, 0, ctx.stream()>>>(
-                y, nc, nr, ns, l.groups, frag.data());
+            const dim3 grid(nr + int(dev::div_ceil(nv, 64 * KS)), l.blocks);
+            kernels::spiral_y_fragments<KS, T8, LO><<<grid, 64 * KS, 0, ctx.stream()>>>(
+                y, nc, nr, ns, l.groups, frag.data(), dev::tissue_view(p), traj.delta_t, voxels.data());
             check_launch("spiral_y_fragments");
         }
         KernelScope scope(ctx, "spiral_hermitian_mfma");

@@ -24,6 +24,7 @@
 #include <string>
 
 #include "compas/device/common.h"
+#include "compas/device/spiral_phasor.h"
 #include "compas/internal.h"
 
 namespace compas {
@@ -72,14 +73,16 @@ __global__ void signal_cartesian_anchors(
     T[size_t(a) * nv + v] = dev::cmul(dev::polar_f(mag, dev::reduce_phase(phi)), tissue.rho(v));
 }
 
-// A[r][v] = m[r][v] * rewind * prephaser * rho (spiral_view.cuh:13-57, signal_kernels.cuh:12-30)
+// A[r][v] = m[r][v] * rewind * prephaser * rho (spiral_view.cuh:13-57, signal_kernels.cuh:12-30);
+// and the voxels' constants for the sums on MFMA, unless nullptr
 __global__ void signal_spiral_factors(
     dev::TissueView tissue, const cfloat* __restrict__ echos, const cfloat* __restrict__ k_start,
-    int nr, int ns, float dt, cfloat* __restrict__ A) {
+    int nr, int ns, float dt, cfloat* __restrict__ A, SpiralVoxel* __restrict__ voxels) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     const int r = blockIdx.y;
     const int nv = tissue.nvoxels;
     if (v >= nv) return;
+    if (voxels != nullptr && r == 0) voxels[v] = spiral_voxel(tissue, dt, v);
     const float R2 = 1.0f / tissue.T2(v);
     const double B0 = tissue.B0(v), x = tissue.x(v);
     const double half = 0.5 * double(ns) * double(dt);
@@ -280,11 +283,15 @@ static Array<cfloat, 3> signal_cartesian(
 }
 
 void spiral_sum(
-    const CompasContext& ctx, const TissueParameters& p, const cfloat* A, const cfloat* Ab, const cfloat* coils,
-    int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out) {
+    const CompasContext& ctx, const TissueParameters& p, const kernels::SpiralVoxel* voxels, const cfloat* A,
+    const cfloat* Ab, const cfloat* coils, int nc, const SpiralTrajectory& t, ContractionPrecision precision,
+    cfloat* out) {
     const int nr = t.nreadouts, ns = t.samples_per_readout;
     if (nc == 0 || nr == 0 || ns == 0) return;
-    if (spiral_sum_mfma(ctx, p, A, Ab, coils, nc, t, precision, out)) return;
+    if (spiral_sum_on_mfma(nc, Ab != nullptr, precision)) {
+        spiral_sum_mfma(ctx, voxels, p.nvoxels, A, Ab, coils, nc, t, precision, out);
+        return;
+    }
     // 8 samples per thread: measured fastest at 4 coils x 1120 x 512 over 50176
     // voxels (24.7 ms, against 35.1 ms for 4 and 30.8 ms for 16, which needs
     // 256 VGPRs and leaves one wave per SIMD)
@@ -314,15 +321,17 @@ static Array<cfloat, 3> signal_spiral(
         return signal;
     }
     auto A = ctx.empty<cfloat, 2>({nr, nv});
+    const ContractionPrecision precision = effective_precision(signal_precision(method));
+    Array<kernels::SpiralVoxel, 1> voxels;
+    if (spiral_sum_on_mfma(nc, false, precision)) voxels = ctx.empty<kernels::SpiralVoxel, 1>({nv});
     {
         KernelScope ks(ctx, "signal_spiral_factors");
         dim3 grid(dev::div_ceil(nv, 256), nr);
         kernels::signal_spiral_factors<<<grid, 256, 0, ctx.stream()>>>(
-            dev::tissue_view(p), echos.data(), t.k_start.data(), nr, ns, t.delta_t, A.data());
+            dev::tissue_view(p), echos.data(), t.k_start.data(), nr, ns, t.delta_t, A.data(), voxels.data());
         check_launch("signal_spiral_factors");
     }
-    spiral_sum(ctx, p, A.data(), nullptr, coils.data(), nc, t, effective_precision(signal_precision(method)),
-               signal.data());
+    spiral_sum(ctx, p, voxels.data(), A.data(), nullptr, coils.data(), nc, t, precision, signal.data());
     return signal;
 }
 

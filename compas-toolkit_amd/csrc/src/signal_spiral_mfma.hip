@@ -71,18 +71,6 @@ __device__ __forceinline__ void split_rows(cfloat w, uint32_t& rh, uint32_t& rl,
     }
 }
 
-__global__ void spiral_voxels(dev::TissueView t, float dt, SpiralVoxel* __restrict__ out) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= t.nvoxels) return;
-    SpiralVoxel o {};
-    o.turns = double(dt) * double(t.B0(v));
-    o.x = t.x(v);
-    o.y = t.y(v);
-    o.T2 = t.T2(v);
-    o.decay = float(-1.4426950408889634 * double(dt) / double(o.T2));  // log2(e)
-    out[v] = o;
-}
-
 typedef float f32x16s __attribute__((ext_vector_type(16)));
 
 // grid (nr, voxel ranges, sample passes), block 64
@@ -245,22 +233,16 @@ __global__ void spiral_sum_reduce(
 
 }  // namespace kernels
 
-Array<kernels::SpiralVoxel, 1> spiral_voxel_table(const CompasContext& ctx, const TissueParameters& p, float dt) {
-    auto voxels = ctx.empty<kernels::SpiralVoxel, 1>({p.nvoxels});
-    KernelScope ks(ctx, "spiral_voxels");
-    kernels::spiral_voxels<<<dev::div_ceil(p.nvoxels, 256), 256, 0, ctx.stream()>>>(dev::tissue_view(p), dt, voxels.data());
-    check_launch("spiral_voxels");
-    return voxels;
+bool spiral_sum_on_mfma(int nc, bool two, ContractionPrecision precision) {
+    return precision != ContractionPrecision::FP32 && nc <= (two ? 4 : 8);  // what the row tiles hold
 }
 
-bool spiral_sum_mfma(
-    const CompasContext& ctx, const TissueParameters& p, const cfloat* A, const cfloat* Ab, const cfloat* coils,
-    int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out) {
-    if (precision == ContractionPrecision::FP32) return false;
+void spiral_sum_mfma(
+    const CompasContext& ctx, const kernels::SpiralVoxel* voxels, int nv, const cfloat* A, const cfloat* Ab,
+    const cfloat* coils, int nc, const SpiralTrajectory& t, ContractionPrecision precision, cfloat* out) {
     const bool two = Ab != nullptr;
-    if (nc > (two ? 4 : 8)) return false;  // more coils than the row tiles hold: the VALU form
     const bool lo = precision == ContractionPrecision::BF16x3 || precision == ContractionPrecision::FP16x3;
-    const int nr = t.nreadouts, ns = t.samples_per_readout, nv = p.nvoxels;
+    const int nr = t.nreadouts, ns = t.samples_per_readout;
     // S = 64 columns for more than 256 samples (half as many rows to generate per
     // column), 32 below; up to 8 S samples a pass
     const int ct = ns > 256 ? 2 : 1;
@@ -278,13 +260,12 @@ bool spiral_sum_mfma(
     const int splits = int(dev::div_ceil(nv, v_chunk));
     const int64_t plane = int64_t(nc) * nr * ns;
     auto partial = ctx.empty<cfloat, 1>({int64_t(splits) * (two ? 2 : 1) * plane});
-    auto voxels = spiral_voxel_table(ctx, p, t.delta_t);
     {
         KernelScope ks(ctx, "spiral_sum_mfma");
         const dim3 grid(nr, splits, passes);
         const auto launch = [&](auto ct_c, auto rt_c, auto two_c, auto lo_c) {
             kernels::spiral_sum_split<decltype(ct_c)::value, decltype(rt_c)::value, decltype(two_c)::value, decltype(lo_c)::value>
-                <<<grid, 64, 0, ctx.stream()>>>(voxels.data(), nv, A, Ab, coils, nc, t.delta_k.data(), nr, ns, tbits,
+                <<<grid, 64, 0, ctx.stream()>>>(voxels, nv, A, Ab, coils, nc, t.delta_k.data(), nr, ns, tbits,
                                                 v_chunk, partial.data());
         };
         const auto with_lo = [&](auto ct_c, auto rt_c, auto two_c) {
@@ -305,7 +286,6 @@ bool spiral_sum_mfma(
     if (two) kernels::spiral_sum_reduce<true><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
     else kernels::spiral_sum_reduce<false><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
     check_launch("spiral_sum_reduce");
-    return true;
 }
 
 }  // namespace compas
