@@ -204,14 +204,17 @@ __global__ void __launch_bounds__(64, 2) spiral_sum_split(
         }
 }
 
-// out[i] = sum over the splits (FP64, in order); with two amplitudes out =
-// first + (s - ns/2) second, s = i % ns
+// out[i] = sum over the splits (FP64, in a fixed order); with two amplitudes out
+// = first + (s - ns/2) second, s = i % ns.  `parts` (a power of two up to 64)
+// lanes share an output, each a range of its splits.
 template<bool TWO>
 __global__ void spiral_sum_reduce(
-    const cfloat* __restrict__ partial, int splits, int64_t n, int ns, cfloat* __restrict__ out) {
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
+    const cfloat* __restrict__ partial, int splits, int parts, int64_t n, int ns, cfloat* __restrict__ out) {
+    for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < n * parts; t += int64_t(gridDim.x) * blockDim.x) {
+        const int64_t i = t / parts;
+        const int part = int(t % parts), per = (splits + parts - 1) / parts;
         double re = 0.0, im = 0.0, bre = 0.0, bim = 0.0;
-        for (int k = 0; k < splits; k++) {
+        for (int k = part * per; k < min(splits, (part + 1) * per); k++) {
             const size_t o = size_t(k) * (TWO ? 2 : 1) * size_t(n) + size_t(i);
             const cfloat p = partial[o];
             re += p.re;
@@ -227,7 +230,11 @@ __global__ void spiral_sum_reduce(
             re = fma(sp, bre, re);
             im = fma(sp, bim, im);
         }
-        out[i] = {float(re), float(im)};
+        for (int off = 1; off < parts; off <<= 1) {
+            re += __shfl_xor(re, off);
+            im += __shfl_xor(im, off);
+        }
+        if (part == 0) out[i] = {float(re), float(im)};
     }
 }
 
@@ -282,9 +289,13 @@ void spiral_sum_mfma(
         check_launch("spiral_sum_mfma");
     }
     KernelScope ks(ctx, "spiral_sum_reduce");
-    const int64_t blocks = std::min<int64_t>(dev::div_ceil(plane, int64_t(256)), 8192);
-    if (two) kernels::spiral_sum_reduce<true><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
-    else kernels::spiral_sum_reduce<false><<<unsigned(blocks), 256, 0, ctx.stream()>>>(partial.data(), splits, plane, ns, out);
+    // a few readouts have few outputs of many splits each: 512 outputs of 2048
+    // splits took 250 us (two amplitudes 500) with one lane to an output
+    int parts = 1;
+    while (parts < 64 && 2 * parts <= splits && plane * parts < (1 << 16)) parts *= 2;
+    const unsigned blocks = unsigned(std::min<int64_t>(dev::div_ceil(plane * parts, int64_t(256)), 8192));
+    if (two) kernels::spiral_sum_reduce<true><<<blocks, 256, 0, ctx.stream()>>>(partial.data(), splits, parts, plane, ns, out);
+    else kernels::spiral_sum_reduce<false><<<blocks, 256, 0, ctx.stream()>>>(partial.data(), splits, parts, plane, ns, out);
     check_launch("spiral_sum_reduce");
 }
 

@@ -52,3 +52,16 @@ def test_products(oracle, nv, nr, ns, nc, method, tol):
     jh = oracle.jacobian_hermitian_spiral(t, traj, coils, wide(m), *[wide(x) for x in d], wide(y), "f64")
     assert rel(ca.compute_jacobian_spiral(m, d, p, tr, coils, v, method=method).collect(), jv) < tol
     assert rel(ca.compute_jacobian_hermitian_spiral(m, d, p, tr, coils, y, method=method).collect(), jh) < tol
+
+
+@pytest.mark.parametrize("nv,nr,ns,nc", [(129, 1, 1, 1), (383, 1, 5, 2), (8191, 1, 3, 1), (8193, 2, 31, 4), (9000, 1, 33, 2)])
+def test_many_voxel_ranges(oracle, nv, nr, ns, nc):
+    """Few outputs of many voxel ranges each: several lanes add up one output, two
+    ranges to one, a last lane with fewer or none."""
+    banner(f"spiral sums over voxel ranges {nv} voxels {nr} x {ns} {nc} coils")
+    t, traj, coils, m, d, v, _, p, tr = case(nv, nr, ns, nc)
+    wide = lambda a: a.astype(np.complex128)  # noqa: E731
+    want = oracle.signal_spiral(t, traj, coils, wide(m), "f64")
+    assert rel(ca.magnetization_to_signal(m, p, tr, coils, method="matmul_fast").collect(), want) < 3e-5
+    jv = oracle.jacobian_spiral(t, traj, coils, wide(m), *[wide(x) for x in d], wide(v), "f64")
+    assert rel(ca.compute_jacobian_spiral(m, d, p, tr, coils, v, method="gemm_fast").collect(), jv) < 3e-5
