@@ -26,9 +26,9 @@
 //     products with conj(m) and conj(dm_p) are done once per readout.
 // Sample blocks of S T and coil groups repeat the two stages within a readout.
 //
-// What bounds it: MFMA (47% of the cycles) and VALU (54%) issue, which overlap
-// little because a barrier per readout keeps the waves of a CU in step, at 1.9
-// GHz.  50176 voxels x 1120 readouts x 512 samples, 4 coils: 14.9 -> 5.6 ms
+// What bounds it: MFMA (47% of the cycles) and VALU (51%) issue, which overlap
+// little because a barrier per readout keeps the waves of a CU in step, at 2.0
+// GHz.  50176 voxels x 1120 readouts x 512 samples, 4 coils: 14.9 -> 5.5 ms
 // against a form that generated every sample's element; 20000 x 500 x 128 854
 // -> 670 us, x 16 452 -> 351 us.
 //

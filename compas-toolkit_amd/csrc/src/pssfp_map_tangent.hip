@@ -16,11 +16,13 @@
 //     entries, 96 VGPRs.  The map of the state itself is shared by the two
 //     fields, three entries to a lane.  Each half advances its own component of
 //     the state and of the tangent; the halves swap components by DPP.
-//   * The sum over slice positions as in pssfp_map.hip.
+//   * The sum over slice positions as in pssfp_map.hip; a workgroup holds 64 or 128
+//     isochromats, so there are several groups, with an FP64 plane each, from
+//     about thirty positions on.
 //
 // What bounds it: FP64 issue.  All four fields and the echoes (two passes) at
-// 3136 voxels x 280 TRs x 35 positions x 25 sub-steps take 1.8 ms (5.6 by
-// sub-steps), 0.54 of them the nodes; at 50176 x 1120 80 ms (271), T1 + T2 at
+// 3136 voxels x 280 TRs x 35 positions x 25 sub-steps take 1.7 ms (5.6 by
+// sub-steps), 0.56 of them the nodes; at 50176 x 1120 82 ms (271), T1 + T2 at
 // 3136 x 280 0.83 (4.3), B1 alone 0.82 (6.7).
 
 #include <algorithm>

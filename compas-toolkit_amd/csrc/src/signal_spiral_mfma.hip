@@ -27,9 +27,9 @@
 //
 // What bounds it: VALU issue (the splits are a third of it) at the clock that
 // the matrix units leave.  At 4 coils x 1120 x 512 over 50176 voxels the signal
-// takes 4.1 ms and J.v 6.8 ms with their amplitude passes (13.1 and 13.8 ms
-// when every sample's element was generated), VALU busy 74% and MFMA 35% of the
-// cycles at 1.8 GHz.  Tried without gain: the next step's generation beside the
+// takes 4.1 ms and J.v 6.7 ms with their amplitude passes (13.1 and 13.8 ms
+// when every sample's element was generated), VALU busy 77% and MFMA 33% of the
+// cycles at 2.1 GHz, with two amplitudes 72% and 43% at 2.0 GHz.  Tried without gain: the next step's generation beside the
 // MFMAs (two LDS buffers, with and without scheduling groups), the two
 // amplitudes in two waves of a workgroup, four waves per SIMD.
 //
