@@ -9,7 +9,8 @@
 //
 // Design (MI355X):
 //   * One isochromat per lane: its 96 Newton coefficients take 192 VGPRs and
-//     stay there for the whole train, two waves per SIMD.  The twelve Horner
+//     stay there for the whole train, two waves per SIMD, without a spill (50176
+//     voxels x 1120 TRs x 35 positions 8.8 ms; 9.3 with 193 spills in the set-up).  The twelve Horner
 //     chains are independent, which hides the FMA latency.  Their common
 //     factors x_n - x_j are the same for every isochromat: wave-uniform, so
 //     scalar loads from the train's table feed SGPR operands.
@@ -157,9 +158,28 @@ __device__ __forceinline__ void pssfp_map_block(
     k.ps *= E2_pr;
     k.pc *= E2_pr;
 
-    // Newton coefficients of the twelve entries
+    // inversion, the alpha/2 pulse with the doubled prephaser, and the first TR
+    // by their sub-steps (pssfp_kernels.cuh:72-75)
+    Vec3d s[1] = {{0.0, 0.0, 0.0}};
+    {
+        const double E1_inv = exp(-double(a.dt_inv) / T1);
+        s[0].z = fma(cos(M_PI * k.B1), E1_inv, 1.0 - E1_inv);
+        const double re = a.RF[0].re, im = a.RF[0].im;
+        pulse(k, grf, a.nRF, -0.5 * re, -0.5 * im, s);
+        double ss, cc;
+        sincos(-(2.0 * double(a.g_pr) * zz) - off_pr, &ss, &cc);
+        rotate_z(s[0], cc, ss);
+        relax3(s[0], k.P1, E2_pr, k.Q1);
+        pulse(k, grf, a.nRF, re, im, s);
+        precess(k, s[0], k.Q1);
+    }
+    // Newton coefficients of the twelve entries.  Those of the first nodes wait in
+    // the lane's slots of the sums until the last node has been through its pulse:
+    // with all in registers the pulse spills, and a kernel with scratch memory is
+    // aborted where the device's memory is taken when it is launched
     const double* train = p.train;
     const double top = train[0];
+    constexpr int WAIT = 2;  // nodes, six slots each of 2 MAP_CHUNK
     double C[MAP_ENTRIES][MAP_NODES];
 #pragma unroll
     for (int j = 0; j < MAP_NODES; j++) {
@@ -180,31 +200,34 @@ __device__ __forceinline__ void pssfp_map_block(
         C[MYZ][j] = m[2].y * odd;
         C[MCX][j] = m[3].x * odd;
         C[MCY][j] = m[3].y * odd;
-    }
+        if (j < WAIT) {
 #pragma unroll
-    for (int o = 1; o < MAP_NODES; o++)
-#pragma unroll
-        for (int j = MAP_NODES - 1; j >= o; j--) {
-            const double inv = 1.0 / (MAP_X[j] - MAP_X[j - o]);
-#pragma unroll
-            for (int e = 0; e < MAP_ENTRIES; e++) C[e][j] = (C[e][j] - C[e][j - 1]) * inv;
+            for (int q = 0; q < 6; q++) {
+                const int slot = 6 * j + q;
+                sums[slot / MAP_CHUNK][slot % MAP_CHUNK][tid] = make_double2(C[2 * q][j], C[2 * q + 1][j]);
+            }
+            asm volatile("" ::: "memory");  // the values live there from here on
         }
-
-    // inversion, the alpha/2 pulse with the doubled prephaser, and the first TR
-    // by their sub-steps (pssfp_kernels.cuh:72-75)
-    Vec3d s[1] = {{0.0, 0.0, 0.0}};
-    {
-        const double E1_inv = exp(-double(a.dt_inv) / T1);
-        s[0].z = fma(cos(M_PI * k.B1), E1_inv, 1.0 - E1_inv);
-        const double re = a.RF[0].re, im = a.RF[0].im;
-        pulse(k, grf, a.nRF, -0.5 * re, -0.5 * im, s);
-        double ss, cc;
-        sincos(-(2.0 * double(a.g_pr) * zz) - off_pr, &ss, &cc);
-        rotate_z(s[0], cc, ss);
-        relax3(s[0], k.P1, E2_pr, k.Q1);
-        pulse(k, grf, a.nRF, re, im, s);
-        precess(k, s[0], k.Q1);
     }
+#pragma unroll
+    for (int j = 0; j < WAIT; j++)
+#pragma unroll
+        for (int q = 0; q < 6; q++) {
+            const int slot = 6 * j + q;
+            const double2 v = sums[slot / MAP_CHUNK][slot % MAP_CHUNK][tid];
+            C[2 * q][j] = v.x;
+            C[2 * q + 1][j] = v.y;
+        }
+    // divided differences, one entry after the other: all at once they spill
+#pragma unroll
+    for (int e = 0; e < MAP_ENTRIES; e++) {
+#pragma unroll
+        for (int o = 1; o < MAP_NODES; o++)
+#pragma unroll
+            for (int j = MAP_NODES - 1; j >= o; j--) C[e][j] = (C[e][j] - C[e][j - 1]) * (1.0 / (MAP_X[j] - MAP_X[j - o]));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
     Vec3d m = s[0];
     // the table's rows are read through the constant address space: the same
     // address in every lane, so scalar loads, each a TR before its use
