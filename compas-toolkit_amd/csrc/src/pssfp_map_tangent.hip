@@ -353,11 +353,15 @@ __device__ __forceinline__ void pssfp_map_tangents_block(const MapTangentArgs& t
 #pragma unroll
     for (int j = 0; j < MAP_NODES; j++) next[j] = row[j];
 
-    const int sum_tr = tid >> 5, sum_t = tid & 31;
     int per = 1;
     while (per < 32 && per * 2 * nvb * NP <= 32) per *= 2;
     const size_t nv_all = size_t(a.tissue.nvoxels), plane = size_t(a.nTR) * nv_all;
     auto write_sums = [&](int n0, int count, int buf) {
+        // formed anew for each chunk: kept, they take the registers that make the
+        // passes of one field spill (pssfp_map.hip says why no kernel may)
+        int lane = tid;
+        asm volatile("" : "+v"(lane));
+        const int sum_tr = lane >> 5, sum_t = lane & 31;
         const int n = n0 + sum_tr;
         for (int w = sum_t / per; w < nvb * NP; w += 32 / per) {
             const int vox = w / NP, k = w % NP;  // plane k: the echoes, then the fields
@@ -418,29 +422,16 @@ __device__ __forceinline__ void pssfp_map_tangents_block(const MapTangentArgs& t
             if (n0 + i > 0) {
                 const double theta = x[0];
                 double e[6], g[6], s[PE];
-                const double h = half ? 1.0 : mz, dh = half ? 0.0 : dz;
 #pragma unroll
                 for (int q = 0; q < PE; q++) s[q] = B[q][MAP_NODES - 1];
 #pragma unroll
                 for (int q = 0; q < 6; q++) g[q] = T[q][MAP_NODES - 1];
-                // one field: its map and then the state's (both together spill;
-                // pssfp_map.hip says why no kernel may)
 #pragma unroll
                 for (int j = MAP_NODES - 2; j >= 0; j--) {
-                    if constexpr (NT > 1) {
 #pragma unroll
-                        for (int q = 0; q < PE; q++) s[q] = fma(s[q], x[1 + j], B[q][j]);
-                    }
+                    for (int q = 0; q < PE; q++) s[q] = fma(s[q], x[1 + j], B[q][j]);
 #pragma unroll
                     for (int q = 0; q < 6; q++) g[q] = fma(g[q], x[1 + j], T[q][j]);
-                }
-                const double gt = fma(g[2], mz, g[3]), gx = fma(g[0], mo, g[1] * mt), gm = g[4] * mo, gh = g[5] * h;
-                if constexpr (NT == 1) {
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int j = MAP_NODES - 2; j >= 0; j--)
-#pragma unroll
-                        for (int q = 0; q < PE; q++) s[q] = fma(s[q], x[1 + j], B[q][j]);
                 }
                 if constexpr (NT == 1) {
 #pragma unroll
@@ -452,10 +443,12 @@ __device__ __forceinline__ void pssfp_map_tangents_block(const MapTangentArgs& t
                         e[3 + q] = quad<0xEE>(s[q]);
                     }
                 }
+                const double h = half ? 1.0 : mz, dh = half ? 0.0 : dz;
                 const double no = fma(theta, fma(e[2], mz, e[3]), fma(e[0], mo, e[1] * mt));
                 const double nz = fma(theta, e[4] * mo, e[5] * h);
-                const double po = fma(theta, fma(e[2], dz, gt), fma(e[0], dox, fma(e[1], dt, gx)));
-                const double pz = fma(theta, fma(e[4], dox, gm), fma(e[5], dh, gh));
+                const double po = fma(theta, fma(e[2], dz, fma(g[2], mz, g[3])),
+                                      fma(e[0], dox, fma(e[1], dt, fma(g[0], mo, g[1] * mt))));
+                const double pz = fma(theta, fma(e[4], dox, g[4] * mo), fma(e[5], dh, g[5] * h));
                 mo = no;
                 mt = quad<0xB1>(no);
                 mz = nz + quad<0xB1>(nz);
