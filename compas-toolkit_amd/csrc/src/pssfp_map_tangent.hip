@@ -357,10 +357,10 @@ __device__ __forceinline__ void pssfp_map_tangents_block(const MapTangentArgs& t
     while (per < 32 && per * 2 * nvb * NP <= 32) per *= 2;
     const size_t nv_all = size_t(a.tissue.nvoxels), plane = size_t(a.nTR) * nv_all;
     auto write_sums = [&](int n0, int count, int buf) {
-        // formed anew for each chunk: kept, they take the registers that make the
-        // passes of one field spill (pssfp_map.hip says why no kernel may)
+        // in a pass of one field formed anew for each chunk: kept, they take the
+        // registers that make it spill (pssfp_map.hip says why no kernel may)
         int lane = tid;
-        asm volatile("" : "+v"(lane));
+        if constexpr (NT == 1) asm volatile("" : "+v"(lane));
         const int sum_tr = lane >> 5, sum_t = lane & 31;
         const int n = n0 + sum_tr;
         for (int w = sum_t / per; w < nvb * NP; w += 32 / per) {
