@@ -24,7 +24,7 @@
 //   * Neighbouring voxel blocks run on one XCD, so that the 8 nv_block bytes a
 //     workgroup writes per TR meet their neighbours' in that XCD's L2.
 //   * What bounds it: FP64 issue.  At 50176 voxels x 1120 TRs x 35 positions the
-//     VALU is busy 75% of the cycles (148 k instructions per wave, 13% of them
+//     VALU is busy 79% of the cycles (148 k instructions per wave, 13% of them
 //     the set-up); the rest is the waits around the chunk sums.
 //   * Whether a train is within MAP_MAX_TYPE is found on the device: the train
 //     lives there and may be rewritten between calls.  The sub-step kernel is

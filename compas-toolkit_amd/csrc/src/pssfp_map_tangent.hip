@@ -22,7 +22,7 @@
 //
 // What bounds it: FP64 issue.  All four fields and the echoes (two passes) at
 // 3136 voxels x 280 TRs x 35 positions x 25 sub-steps take 1.7 ms (5.6 by
-// sub-steps), 0.56 of them the nodes; at 50176 x 1120 82 ms (271), T1 + T2 at
+// sub-steps), 0.56 of them the nodes; at 50176 x 1120 83 ms (271), T1 + T2 at
 // 3136 x 280 0.83 (4.3), B1 alone 0.82 (6.7).
 
 #include <algorithm>
